@@ -50,9 +50,11 @@ __device__ __forceinline__ float quick_fill(float rec, float ion) {
 }
 
 // get_HIIbubbles.c:339-349: centre iff ion > 0 and (rec <= 0 or
-// ion/rec >= 1); for rec > 0 the FP64 quotient test equals ion >= rec.
+// ion/rec >= 1); for rec > 0 the FP64 quotient test equals ion >= rec.  With
+// ion > 0 a rec <= 0 never exceeds ion, and a NaN rec compares false, so "not
+// (ion < rec)" covers both cases in one comparison without a branch.
 __device__ __forceinline__ bool is_centre(float rec, float ion) {
-  return (ion > 0.0f) && (!(rec > 0.0f) || ion >= rec);
+  return (ion > 0.0f) & !(ion < rec);
 }
 
 }  // namespace sf21

@@ -20,8 +20,22 @@
 
 namespace sf21 {
 
+// The products and sums of the transforms are spelled out as roundings and
+// fused multiply-adds instead of being left to the compiler's contraction,
+// which chooses by basic block: the centre test is discontinuous, so the same
+// line has to come out bit for bit in every kernel that carries it.
 __device__ __forceinline__ float2 cmul(float2 a, float2 b) {
   return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+}
+// a*b rounded: never part of a fused multiply-add
+__device__ __forceinline__ float mul_rounded(float a, float b) {
+#pragma clang fp contract(off)
+  return a * b;
+}
+// cmul with its roundings spelled out: the form the compiler gives cmul in
+// every radix-8 plan (each component's a*b.y product rounded, the other fused)
+__device__ __forceinline__ float2 cmul_fixed(float2 a, float2 b) {
+  return make_float2(fmaf(a.x, b.x, -mul_rounded(a.y, b.y)), fmaf(a.y, b.x, mul_rounded(a.x, b.y)));
 }
 __device__ __forceinline__ float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
 __device__ __forceinline__ float2 csub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
@@ -31,12 +45,14 @@ __device__ __forceinline__ float2 mul_si(float2 a) {
   return SIGN > 0 ? make_float2(-a.y, a.x) : make_float2(a.y, -a.x);
 }
 
-// In-register DFTs, y_k = sum_n x_n exp(SIGN*2*pi*i*n*k/R).
-template <int R, int SIGN>
+// In-register DFTs, y_k = sum_n x_n exp(SIGN*2*pi*i*n*k/R).  ROUND: the
+// subtracted half of the outputs takes its products rounded instead of fused
+// (the centre-test pass's last stage).
+template <int R, int SIGN, bool ROUND = false>
 struct Dft;
 
-template <int SIGN>
-struct Dft<2, SIGN> {
+template <int SIGN, bool ROUND>
+struct Dft<2, SIGN, ROUND> {
   static __device__ __forceinline__ void run(float2* a) {
     float2 t = a[1];
     a[1] = csub(a[0], t);
@@ -44,8 +60,8 @@ struct Dft<2, SIGN> {
   }
 };
 
-template <int SIGN>
-struct Dft<4, SIGN> {
+template <int SIGN, bool ROUND>
+struct Dft<4, SIGN, ROUND> {
   static __device__ __forceinline__ void run(float2* a) {
     float2 t0 = cadd(a[0], a[2]), t1 = csub(a[0], a[2]);
     float2 t2 = cadd(a[1], a[3]), t3 = mul_si<SIGN>(csub(a[1], a[3]));
@@ -56,8 +72,8 @@ struct Dft<4, SIGN> {
   }
 };
 
-template <int SIGN>
-struct Dft<8, SIGN> {
+template <int SIGN, bool ROUND>
+struct Dft<8, SIGN, ROUND> {
   static __device__ __forceinline__ void run(float2* a) {
     const float h = 0.70710678118654752440f;
     float2 e[4] = {a[0], a[2], a[4], a[6]};
@@ -65,33 +81,47 @@ struct Dft<8, SIGN> {
     Dft<4, SIGN>::run(e);
     Dft<4, SIGN>::run(o);
     // o[k] *= exp(SIGN*2*pi*i*k/8)
-    float2 o1 = o[1], o3 = o[3];
-    o[1] = make_float2(h * (o1.x - SIGN * o1.y), h * (o1.y + SIGN * o1.x));
-    o[2] = mul_si<SIGN>(o[2]);
-    o[3] = make_float2(h * (-o3.x - SIGN * o3.y), h * (-o3.y + SIGN * o3.x));
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      a[k] = cadd(e[k], o[k]);
-      a[k + 4] = csub(e[k], o[k]);
+    const float2 q2 = mul_si<SIGN>(o[2]);
+    a[0] = cadd(e[0], o[0]);
+    a[4] = csub(e[0], o[0]);
+    a[2] = cadd(e[2], q2);
+    a[6] = csub(e[2], q2);
+    // the odd outputs' rotations by (2k+1) pi/4 are h times these
+    const float2 q1 = make_float2(o[1].x - SIGN * o[1].y, o[1].y + SIGN * o[1].x);
+    const float2 q3 = make_float2(-o[3].x - SIGN * o[3].y, -o[3].y + SIGN * o[3].x);
+    a[1] = make_float2(fmaf(h, q1.x, e[1].x), fmaf(h, q1.y, e[1].y));
+    a[3] = make_float2(fmaf(h, q3.x, e[3].x), fmaf(h, q3.y, e[3].y));
+    if constexpr (ROUND) {
+      a[5] = make_float2(e[1].x - mul_rounded(h, q1.x), e[1].y - mul_rounded(h, q1.y));
+      a[7] = make_float2(e[3].x - mul_rounded(h, q3.x), e[3].y - mul_rounded(h, q3.y));
+    } else {
+      a[5] = make_float2(fmaf(-h, q1.x, e[1].x), fmaf(-h, q1.y, e[1].y));
+      a[7] = make_float2(fmaf(-h, q3.x, e[3].x), fmaf(-h, q3.y, e[3].y));
     }
   }
 };
 
-template <int SIGN>
-struct Dft<3, SIGN> {
+template <int SIGN, bool ROUND>
+struct Dft<3, SIGN, ROUND> {
   static __device__ __forceinline__ void run(float2* a) {
     const float c = -0.5f, s = SIGN * 0.86602540378443864676f;
     float2 t1 = cadd(a[1], a[2]), t2 = csub(a[1], a[2]);
     float2 m = make_float2(a[0].x + c * t1.x, a[0].y + c * t1.y);
-    float2 r = make_float2(-s * t2.y, s * t2.x);
-    a[0] = cadd(a[0], t1);
-    a[1] = cadd(m, r);
-    a[2] = csub(m, r);
+    if constexpr (ROUND) {
+      a[0] = cadd(a[0], t1);
+      a[1] = make_float2(fmaf(-s, t2.y, m.x), fmaf(s, t2.x, m.y));
+      a[2] = make_float2(m.x + mul_rounded(s, t2.y), m.y - mul_rounded(s, t2.x));
+    } else {
+      float2 r = make_float2(-s * t2.y, s * t2.x);
+      a[0] = cadd(a[0], t1);
+      a[1] = cadd(m, r);
+      a[2] = csub(m, r);
+    }
   }
 };
 
-template <int SIGN>
-struct Dft<5, SIGN> {
+template <int SIGN, bool ROUND>
+struct Dft<5, SIGN, ROUND> {
   static __device__ __forceinline__ void run(float2* a) {
     const float c1 = 0.30901699437494742410f, c2 = -0.80901699437494742410f;
     const float s1 = SIGN * 0.95105651629515357212f, s2 = SIGN * 0.58778525229247312917f;
@@ -133,6 +163,18 @@ __device__ __forceinline__ void st_stream(float2* p, float2 a) {
 // clobber pins every LDS access of an exchange on its side of the barrier.
 __device__ __forceinline__ void lds_pin() { asm volatile("" ::: "memory"); }
 
+// The synchronisation of an LDS exchange.  WAVE: the line's threads all sit
+// in one wave (lines along p: L/E <= 64 threads, a power of two, consecutive
+// lanes).  LDS operations of one wave complete in issue order, so only the
+// compiler has to be held, and the block's waves run independently.  Lines
+// spread over several waves (columns) take the block barrier.
+template <bool WAVE>
+__device__ __forceinline__ void exchange_sync() {
+  lds_pin();
+  if constexpr (WAVE) __builtin_amdgcn_wave_barrier();
+  else __syncthreads();
+}
+
 // Returns v unchanged but opaque to the optimiser.  Used on the lane index
 // at the top of radius loops: without it the compiler hoists every FFT
 // stage's LDS and twiddle addresses out of the loop and keeps them live in
@@ -141,6 +183,15 @@ __device__ __forceinline__ void lds_pin() { asm volatile("" ::: "memory"); }
 __device__ __forceinline__ int opaque_lane(int v) {
   asm volatile("" : "+v"(v));
   return v;
+}
+
+// A wave-uniform pointer kept in scalar registers: the access adds the lane's
+// 32-bit offset in its own address unit, where the compiler would otherwise
+// fold base and offset into 64-bit vector additions per access.
+template <class T>
+__device__ __forceinline__ T* uniform_ptr(T* p) {
+  asm("" : "+s"(p));
+  return p;
 }
 
 // LDS index padding: one slot every 8 breaks the stride-R write pattern of
@@ -192,7 +243,7 @@ struct StageSlots {
 // Index arithmetic is unsigned (lanes are non-negative), and where the
 // thread's butterflies b share k = t mod NS (TPL a multiple of NS) the LDS
 // slots of every b and r are one per-thread base plus compile-time offsets.
-template <int L, int E, int SIGN, int NS, int R, int... REST>
+template <int L, int E, int SIGN, bool WAVE, bool ROUND, int NS, int R, int... REST>
 __device__ __forceinline__ void stages(float2 (&v)[E], float* sre, float* sim, int t,
                                        const float2* __restrict__ tw) {
   constexpr int TPL = L / E;
@@ -220,7 +271,7 @@ __device__ __forceinline__ void stages(float2 (&v)[E], float* sre, float* sim, i
         a[r] = cmul(a[r], w);
       }
     }
-    Dft<R, SIGN>::run(a);
+    Dft<R, SIGN, ROUND && LAST>::run(a);
     if constexpr (LAST) {
 #pragma unroll
       for (int r = 0; r < R; ++r) v[b + r * NB] = a[r];
@@ -243,41 +294,157 @@ __device__ __forceinline__ void stages(float2 (&v)[E], float* sre, float* sim, i
     }
   }
   if constexpr (!LAST) {
-    lds_pin();
-    __syncthreads();
+    exchange_sync<WAVE>();
     const unsigned pt = lds_pad_u(ut);
 #pragma unroll
     for (int m = 0; m < E; ++m) {
       const unsigned o = (TPL % 8 == 0) ? pt + (unsigned)(m * (TPL + TPL / 8)) : lds_pad_u(ut + TPL * m);
       v[m] = make_float2(sre[o], sim[o]);
     }
-    lds_pin();
-    __syncthreads();
-    stages<L, E, SIGN, NS * R, REST...>(v, sre, sim, t, tw);
+    exchange_sync<WAVE>();
+    stages<L, E, SIGN, WAVE, ROUND, NS * R, REST...>(v, sre, sim, t, tw);
   }
 }
 
-template <int L, int E, int SIGN, int... Rs>
+template <int L, int E, int SIGN, bool WAVE, bool ROUND, int... Rs>
 __device__ __forceinline__ void line_fft_impl(float2 (&v)[E], float* sre, float* sim, int t,
                                               const float2* __restrict__ tw, RadixList<Rs...>) {
-  stages<L, E, SIGN, 1, Rs...>(v, sre, sim, t, tw);
+  static_assert(!WAVE || (L / E <= 64 && 64 % (L / E) == 0), "a wave must hold whole lines");
+  stages<L, E, SIGN, WAVE, ROUND, 1, Rs...>(v, sre, sim, t, tw);
+}
+
+// Twiddles of a thread's line held in registers, in the order of the stages:
+// for radius loops.  A twiddle load inside such a loop waits for every
+// earlier load and store of the wave (they retire in order) -- the filtered
+// lines' stores, the next line's prefetch -- and the compiler does not move
+// it out by itself past the exchanges' memory clobbers.
+template <int L, int E, int NS, int R, int... REST>
+constexpr int twiddle_count() {
+  constexpr int own = NS == 1 ? 0 : ((L / E) % NS == 0 ? 1 : E / R) * (R - 1);
+  if constexpr (sizeof...(REST) == 0) return own;
+  else return own + twiddle_count<L, E, NS * R, REST...>();
+}
+
+template <int L, int E, int OFF, int NS, int R, int... REST>
+__device__ __forceinline__ void twiddle_load(float2* w, int t, const float2* __restrict__ tw) {
+  constexpr int TPL = L / E, NB = (NS == 1) ? 0 : (TPL % NS == 0 ? 1 : E / R);
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    const unsigned ks = (((unsigned)t + TPL * b) % NS) * (unsigned)(L / (NS * R));
+#pragma unroll
+    for (int r = 1; r < R; ++r) w[OFF + b * (R - 1) + r - 1] = tw[ks * r];
+  }
+  if constexpr (sizeof...(REST) > 0)
+    twiddle_load<L, E, OFF + NB * (R - 1), NS * R, REST...>(w, t, tw);
+}
+
+template <int L, int E, class List>
+struct TwRegsOf;
+template <int L, int E, int... Rs>
+struct TwRegsOf<L, E, RadixList<Rs...>> {
+  static constexpr int kCount = twiddle_count<L, E, 1, Rs...>();
+  float2 w[kCount > 0 ? kCount : 1];
+  __device__ __forceinline__ void load(int t, const float2* __restrict__ tw) {
+    twiddle_load<L, E, 0, 1, Rs...>(w, t, tw);
+  }
+};
+template <int L, int E>
+using TwRegs = TwRegsOf<L, E, typename Radices<L>::type>;
+
+// The same stages with the twiddles from registers (TWREG: wreg, see TwRegs)
+// or from a table tw that a radius loop keeps in LDS, and the twiddle products
+// in the fixed form.  Not for the forward transforms of the sides with a
+// radix 3: there the compiler gives some products of stages() another form.
+template <int L, int E, int SIGN, bool WAVE, bool ROUND, bool TWREG, int OFF, int NS, int R, int... REST>
+__device__ __forceinline__ void loop_stages(float2 (&v)[E], float* sre, float* sim, int t,
+                                            const float2* wreg, const float2* tw) {
+  constexpr int TPL = L / E, NB = E / R;
+  constexpr bool LAST = sizeof...(REST) == 0;
+  constexpr bool kUniformK = TPL % NS == 0;
+  constexpr bool kFastW = kUniformK && StageSlots<NS, R>::kConst && (TPL * R) % 8 == 0;
+  const unsigned ut = (unsigned)t;
+  const unsigned k0 = ut % NS;
+  const unsigned pbase0 = lds_pad_u((ut / NS) * NS * R + k0);
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    const unsigned j = ut + TPL * b;
+    const unsigned k = kUniformK ? k0 : j % NS;
+    float2 a[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) a[r] = v[b + r * NB];
+    if constexpr (NS > 1) {
+      const unsigned ks = k * (unsigned)(L / (NS * R));
+#pragma unroll
+      for (int r = 1; r < R; ++r) {
+        float2 w = TWREG ? wreg[OFF + (kUniformK ? 0 : b) * (R - 1) + r - 1] : tw[ks * r];
+        if (SIGN > 0) w.y = -w.y;
+        a[r] = cmul_fixed(a[r], w);
+      }
+    }
+    Dft<R, SIGN, ROUND && LAST>::run(a);
+    if constexpr (LAST) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[b + r * NB] = a[r];
+    } else {
+      const unsigned pb = pbase0 + (unsigned)(b * (TPL * R + (TPL * R) / 8));
+      const unsigned base = (j / NS) * NS * R + k;
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const unsigned o = kFastW ? pb + StageSlots<NS, R>::off(r) : lds_pad_u(base + r * NS);
+        sre[o] = a[r].x;
+        sim[o] = a[r].y;
+      }
+    }
+  }
+  if constexpr (!LAST) {
+    exchange_sync<WAVE>();
+    const unsigned pt = lds_pad_u(ut);
+#pragma unroll
+    for (int m = 0; m < E; ++m) {
+      const unsigned o = (TPL % 8 == 0) ? pt + (unsigned)(m * (TPL + TPL / 8)) : lds_pad_u(ut + TPL * m);
+      v[m] = make_float2(sre[o], sim[o]);
+    }
+    exchange_sync<WAVE>();
+    constexpr int kOwn = NS == 1 ? 0 : (kUniformK ? 1 : NB) * (R - 1);
+    loop_stages<L, E, SIGN, WAVE, ROUND, TWREG, OFF + kOwn, NS * R, REST...>(v, sre, sim, t, wreg, tw);
+  }
+}
+
+template <int L, int E, int SIGN, bool WAVE, bool ROUND, bool TWREG, int... Rs>
+__device__ __forceinline__ void loop_fft_impl(float2 (&v)[E], float* sre, float* sim, int t,
+                                              const float2* wreg, const float2* tw, RadixList<Rs...>) {
+  static_assert(!WAVE || (L / E <= 64 && 64 % (L / E) == 0), "a wave must hold whole lines");
+  loop_stages<L, E, SIGN, WAVE, ROUND, TWREG, 0, 1, Rs...>(v, sre, sim, t, wreg, tw);
+}
+
+// A line's transform inside a radius loop; twiddles from a table in LDS or
+// from registers.
+template <int L, int E, int SIGN, bool WAVE = false, bool ROUND = false>
+__device__ __forceinline__ void loop_fft(float2 (&v)[E], float* sre, float* sim, int t,
+                                         const float2* tw) {
+  loop_fft_impl<L, E, SIGN, WAVE, ROUND, false>(v, sre, sim, t, nullptr, tw, typename Radices<L>::type{});
+}
+template <int L, int E, int SIGN, bool WAVE = false, bool ROUND = false>
+__device__ __forceinline__ void loop_fft(float2 (&v)[E], float* sre, float* sim, int t,
+                                         const TwRegs<L, E>& w) {
+  loop_fft_impl<L, E, SIGN, WAVE, ROUND, true>(v, sre, sim, t, w.w, nullptr, typename Radices<L>::type{});
 }
 
 // Line transform with E values per thread (every radix of the size's plan
 // must divide E): E = 16 halves the threads per line and doubles the work
 // between the exchanges' barriers.
-template <int L, int E, int SIGN>
+template <int L, int E, int SIGN, bool WAVE = false, bool ROUND = false>
 __device__ __forceinline__ void line_fft_e(float2 (&v)[E], float* sre, float* sim, int t,
                                            const float2* __restrict__ tw) {
-  line_fft_impl<L, E, SIGN>(v, sre, sim, t, tw, typename Radices<L>::type{});
+  line_fft_impl<L, E, SIGN, WAVE, ROUND>(v, sre, sim, t, tw, typename Radices<L>::type{});
 }
 
-// Full line transform.  Every thread of the block must call it (it contains
-// block barriers), including threads whose line is out of range.
-template <int L, int SIGN>
+// Full line transform.  Every thread of the block must call it (without WAVE
+// it contains block barriers), including threads whose line is out of range.
+template <int L, int SIGN, bool WAVE = false>
 __device__ __forceinline__ void line_fft(float2 (&v)[Plan<L>::E], float* sre, float* sim, int t,
                                          const float2* __restrict__ tw) {
-  line_fft_impl<L, Plan<L>::E, SIGN>(v, sre, sim, t, tw, typename Radices<L>::type{});
+  line_fft_impl<L, Plan<L>::E, SIGN, WAVE, false>(v, sre, sim, t, tw, typename Radices<L>::type{});
 }
 
 // Signed frequency index as the reference folds it (get_HIIbubbles.c:309-315):

@@ -66,17 +66,38 @@ void launch_fwd_rows(int n, const float* a, const float* b, const float* c, Cell
 // values per thread instead of the size's default (sizes 128, 256, 512);
 // bit 1: blocks walk 8 tiles, prefetching the next (tile 16, or 16 and 32 wide);
 // bit 2: non-temporal loads and stores; bit 3 (axis 0, width n): the array
-// is in the 16-column tile layout -- each (i, 16 p columns) tile an n x 16
-// block, element (i, j, p) at i n^2 + (p/16) 16 n + 16 j + p%16
+// is in the 16-column tile layout (t16_tile in kernels_fused.hip)
 void launch_cols(int n, int width, int axis, int sign, const float2* in, float2* out,
                  int nbatch, long bstride, const float2* tw, hipStream_t s, int tile = 16,
                  int variant = 0);
-// jpair: one block per mirror pair of i-lines (kj, n - kj), sharing W
-// (tile 8 or 16, weights evaluated in the kernel); t16: u in the 16-column
-// tile layout of launch_cols (the p pass then reads it with t16 as well)
+// Top-hat weights of the filter passes, all radii of the ladder.  mode 0:
+// lut, the FP64 table per integer |k|^2 (mlut entries per radius); mode 1:
+// FP32, from the weight table or, without one, evaluated in the pass from
+// kappa = dk R as hi + lo.
+struct FilterW {
+  int mode;
+  const float* lut;
+  long mlut;
+  const float* table;
+  const float2* kappa;
+};
+// floats of one radius of the weight table: [fj][p/16][fi][p%16]
+constexpr long wtab_radius(int n) { return (long)(n / 2 + 1) * (n / 2 + 1) * ((n + 15) / 16 * 16); }
+void launch_w_table(int n, int nr, const float2* kappa, float* wt, hipStream_t s);
+// radii rb .. rb + nrad - 1 of the ladder; mirror: the block order that runs
+// the i-lines kj and n - kj, which share their weights, together on one XCD;
+// t16: u in the 16-column tile layout of launch_cols (the p pass then reads
+// it with t16 as well)
 void launch_filter_i(int n, const float2* spec, float2* u, int nrad, long ustride,
-                     const float* wlut, long m_lut, const float2* kappa, const float2* tw,
-                     hipStream_t s, int tile, int wmode, bool jpair = false, bool t16 = false);
+                     const FilterW& w, int rb, const float2* tw, hipStream_t s, int tile,
+                     bool mirror = false, bool t16 = false);
+// sides whose j and p inverses and centre test run plane by plane (u in the
+// natural layout); prepare allows the blocks' LDS on the current device
+bool plane_side(int n);
+bool plane_prepare(int n);
+void launch_plane_crit(int n, const float2* u, int nrad, long ustride, const int* d2max,
+                       const float* bal, int* wmap, float2* dbg, float2* keep, const float2* tw,
+                       hipStream_t s);
 void launch_inv_rows_crit(int n, const float2* v, int nrad, long vstride, const int* d2max,
                           const float* bal, int* wmap, float2* dbg, hipStream_t s,
                           const float2* tw, bool wide = false,

@@ -119,6 +119,30 @@ __global__ __launch_bounds__(256) void k_fwd_rows(const float* __restrict__ a,
 }
 
 // ------------------------------------------------------------------------
+// Tile layout of the per-radius buffer on the sides from 192: each (i, 16
+// adjacent p) tile one contiguous L x 16 block, the tiles of one column group
+// behind each other along i; element (i, j, p) at t16_tile(i, p/16) + 16 j +
+// p%16.  The j pass reads and writes whole blocks.  The i pass's line of one
+// column group lies within 32 MiB at 512 (16 pages of 2 MiB) instead of one
+// page per position over the whole 1 GiB box; a row of the p pass takes one
+// page per tile instead.  512^3 slice, 47 radii in one batch: filter pass
+// 12.9 -> 11.2 ms, p pass 7.9 -> 8.3 ms against tiles ordered by i first;
+// groups of 8 i in between gave 12.1 and 8.0 ms.
+// ------------------------------------------------------------------------
+template <int L>
+__device__ __forceinline__ long t16_tile(int i, int pt) {
+  return ((long)pt * L + i) * (16 * L);
+}
+// Block q of a pass over that layout, in memory order: outer i and first
+// column of its TILE columns.
+template <int L, int TILE>
+__device__ __forceinline__ void t16_block(int q, int& i, int& col) {
+  constexpr int S = TILE < 16 ? 16 / TILE : 1, W = TILE < 16 ? 16 : TILE;
+  i = q / S % L;
+  col = q / (S * L) * W + q % S * TILE;
+}
+
+// ------------------------------------------------------------------------
 // Strided complex transform along j (axis 0) or i (axis 1) of an
 // L x L x width array; TILE adjacent columns per block (128 B runs).
 // blockIdx.y selects one of several arrays spaced bstride apart.
@@ -132,8 +156,9 @@ __global__ __launch_bounds__(TILE*(L / E)) void k_cols(const float2* in, float2*
   __shared__ float lds[TILE * 2 * LdsLine<L>::kFloats];
   const int c = threadIdx.x % TILE, t = threadIdx.x / TILE;
   const int ntile = (width + TILE - 1) / TILE;
-  const int outer = blockIdx.x / ntile;
-  const int col = (blockIdx.x % ntile) * TILE + c;
+  int outer = blockIdx.x / ntile, col = (blockIdx.x % ntile) * TILE;
+  if (axis == 2) t16_block<L, TILE>(blockIdx.x, outer, col);
+  col += c;
   const bool ok = col < width;
   long base, stride;
   if (axis == 0) {
@@ -143,7 +168,7 @@ __global__ __launch_bounds__(TILE*(L / E)) void k_cols(const float2* in, float2*
     base = (long)outer * width + col;
     stride = (long)L * width;
   } else {  // 2: along j in the 16-column tile layout (width L)
-    base = (long)outer * L * width + (long)(col >> 4) * (L * 16) + (col & 15);
+    base = t16_tile<L>(outer, col >> 4) + (col & 15);
     stride = 16;
   }
   base += (long)blockIdx.y * bstride;
@@ -195,12 +220,13 @@ __global__ __launch_bounds__(TILE*(L / E)) void k_cols_pipe(const float2* in, fl
   auto origin = [&](long q) -> long {
     const long y = q / ((long)ntile * L);
     const long rem = q - y * ((long)ntile * L);
-    const int outer = (int)(rem / ntile);
-    const int col = (int)(rem % ntile) * TILE + c;
+    int outer = (int)(rem / ntile), col = (int)(rem % ntile) * TILE;
+    if (axis == 2) t16_block<L, TILE>((int)rem, outer, col);
+    col += c;
     if (col >= width) return -1;
     const long b = axis == 0   ? (long)outer * L * width + col
                    : axis == 1 ? (long)outer * width + col
-                               : (long)outer * L * width + (long)(col >> 4) * (L * 16) + (col & 15);
+                               : t16_tile<L>(outer, col >> 4) + (col & 15);
     return b + y * bstride;
   };
   float2 cur[E], nxt[E];
@@ -241,45 +267,130 @@ __global__ __launch_bounds__(TILE*(L / E)) void k_cols_pipe(const float2* in, fl
 }
 
 // ------------------------------------------------------------------------
-// Per radius batch: forward along i of the (p, j)-transformed spectrum,
-// top-hat filter W(|k| R) for each radius (get_HIIbubbles.c:305-322; W from
-// an FP64 table indexed by the integer |k|^2, rounded to float), inverse
-// along i.  The forward spectrum along i never leaves the registers.
+// Top-hat weights of every radius, laid out as the filter passes read them:
+// wt[r][fj][p/16][fi][p%16] (fj, fi <= n/2 the folded frequencies along j and
+// i): a block's weights of one radius are one contiguous piece of whole cache
+// lines.  The same function of the same integer |k|^2 as an evaluation in the
+// filter pass, so the same values; computed once per context.
 // ------------------------------------------------------------------------
-// JPAIR: a block takes the lines at kj and L - kj (kj = 1 + block row, up
-// to L/2 - 1) of the same p columns, which share every W value (|k|^2
-// depends on kj^2 only): one W evaluation serves two lines, whose inverse
-// transforms run one after the other through the same LDS region.  Without
-// JPAIR a block takes the line kj = block row * kj_step (kj_step L/2 covers
-// the unpaired lines 0 and L/2).
-template <int L, int TILE, bool WTAB, bool JPAIR = false>
+__global__ __launch_bounds__(256) void k_w_table(int n, const float2* __restrict__ kappa,
+                                                 float* __restrict__ wt) {
+  const int H = n / 2 + 1, ct = (n + 15) / 16;
+  const int pt = blockIdx.x, fj = blockIdx.y, r = blockIdx.z;
+  float* __restrict__ blk = wt + (((long)r * H + fj) * ct + pt) * (H * 16);
+  for (int e = threadIdx.x; e < H * 16; e += blockDim.x) {
+    const int fi = e >> 4, p = pt * 16 + (e & 15);
+    blk[e] = w_tophat_k(kappa[r], fj * fj + fi * fi + fold_sq(p, n));
+  }
+}
+
+// ------------------------------------------------------------------------
+// Per radius batch: forward along i of the (p, j)-transformed spectrum,
+// top-hat filter W(|k| R) for each radius (get_HIIbubbles.c:305-322), inverse
+// along i.  The forward spectrum along i never leaves the registers.
+// Block: TILE columns of one line kj.  mirror: the lines kj and L - kj, which
+// read the same weights, 8 blocks apart -- on one XCD and running together,
+// the second reads them from its L2.  blockIdx.y: groups of rper radii, so
+// that small boxes fill the GPU.
+// Sides 256 and 512 hold 16 values per thread: at 512 two blocks of 512
+// threads share a CU (78 KiB of LDS, 128 VGPRs each) and fill each other's
+// exchange barriers.
+// Bound: the stores (512^3: 50.5 GB per slice, with the table's 6.4 GB 5.2
+// TB/s).  512^3, 47 radii, per slice: 14.2 ms with the weights evaluated in
+// the loop (a third of its VALU instructions), twiddle loads in it and two
+// lines per 1024-thread block; 17.9 ms with a table in folded order (half
+// cache lines); 14.8 ms with this one; 13.1 ms with the buffer's tiles ordered
+// along i; 11.2 ms with the whole ladder in one batch.  Mirror lines together:
+// 1.63 -> 1.50 ms at 256, 13.8 -> 13.1 ms at 512.
+// ------------------------------------------------------------------------
+template <int L>
+struct FilterE {
+  static constexpr int kE = L >= 256 ? 16 : Plan<L>::E;
+};
+
+template <int L, int TILE>
+__global__ __launch_bounds__(TILE*(L / FilterE<L>::kE)) void k_filter_tab(
+    const float2* __restrict__ spec, float2* __restrict__ u, int nrad, int rper, long ustride,
+    const float* __restrict__ wt, const float2* __restrict__ tw, int mirror, int t16) {
+  constexpr int E = FilterE<L>::kE, TPL = L / E, NT = L / TILE, H = L / 2 + 1;
+  __shared__ float lds[TILE * 2 * LdsLine<L>::kFloats];
+  __shared__ float2 twl[L];  // for the radius loop: see TwRegs
+  for (int q = threadIdx.x; q < L; q += TILE * TPL) twl[q] = tw[q];
+  const int c = threadIdx.x % TILE, t = threadIdx.x / TILE;
+  int kj = blockIdx.x / NT, tile = blockIdx.x % NT;
+  if (mirror) {
+    const int pair = (blockIdx.x >> 4) * 8 + (blockIdx.x & 7);
+    const int row = pair / NT;
+    tile = pair % NT;
+    kj = (blockIdx.x & 8) ? (row == 0 ? L / 2 : L - row) : row;
+  }
+  const int p0 = tile * TILE, kp = p0 + c;
+  float* sre = lds + c * 2 * LdsLine<L>::kFloats;
+  float* sim = sre + LdsLine<L>::kFloats;
+  // element e of this line sits at line[e * L * L] (32-bit offsets: L^3 < 2^31)
+  float2 z[E];
+  const float2* __restrict__ src = spec + (long)kj * L + p0;
+#pragma unroll
+  for (int m = 0; m < E; ++m) z[m] = (src + m * TPL * (L * L))[t * (L * L) + c];
+  __syncthreads();
+  if constexpr (E == Plan<L>::E) line_fft<L, -1>(z, sre, sim, t, tw);
+  else loop_fft<L, E, -1>(z, sre, sim, t, twl);
+  // weights of positions t + TPL m: frequency t + TPL m below L/2, its mirror
+  // L - t - TPL m above (both L/2 at the middle)
+  const unsigned wlo = t * 16 + (kp & 15), whi = (TPL - t) * 16 + (kp & 15);
+  const int r0 = blockIdx.y * rper, r1 = min(r0 + rper, nrad);
+  constexpr long kWRadius = (long)H * (L / 16) * (H * 16);
+  const float* __restrict__ wr =
+      wt + r0 * kWRadius + ((long)(kj <= L / 2 ? kj : L - kj) * (L / 16) + (p0 >> 4)) * (H * 16);
+  float wv[E];
+  auto weights = [&]() {
+#pragma unroll
+    for (int m = 0; m < E; ++m)
+      wv[m] = m < E / 2 ? uniform_ptr(wr + m * TPL * 16)[wlo]
+                        : uniform_ptr(wr + (L - TPL * (m + 1)) * 16)[whi];
+  };
+  weights();
+#pragma unroll 1
+  for (int r = r0; r < r1; ++r) {
+    const int tl = opaque_lane(t);
+    float2 v[E];
+#pragma unroll
+    for (int m = 0; m < E; ++m) v[m] = make_float2(z[m].x * wv[m], z[m].y * wv[m]);
+    wr += kWRadius;
+    if (r + 1 < r1) weights();  // in flight during the transform
+    loop_fft<L, E, +1>(v, sre, sim, tl, twl);
+    const int si = t16 ? 16 * L : L * L;  // stride along i
+    float2* __restrict__ dst =
+        u + (long)r * ustride + (t16 ? t16_tile<L>(0, p0 >> 4) + kj * 16 : (long)kj * L + p0);
+    const unsigned o = tl * si + (t16 ? (kp & 15) : c);
+#pragma unroll
+    for (int m = 0; m < E; ++m) st_stream(uniform_ptr(dst + m * TPL * si) + o, v[m]);
+  }
+}
+
+// The filter pass without the weight table: weights from the FP64 table per
+// integer |k|^2 (WTAB), or evaluated per position (no memory for the
+// table).  One line per block.
+template <int L, int TILE, bool WTAB>
 __global__ __launch_bounds__(TILE*(L / Plan<L>::E)) void k_filter_i(
     const float2* __restrict__ spec, float2* __restrict__ u, int nrad, long ustride,
     const float* __restrict__ wlut, long mlut, const float2* __restrict__ kappa,
-    const float2* __restrict__ tw, int kj_step, int t16) {
+    const float2* __restrict__ tw, int t16) {
   constexpr int E = Plan<L>::E, TPL = L / E, NT = L / TILE;
-  constexpr int NL = JPAIR ? 2 : 1;
   __shared__ float lds[TILE * 2 * LdsLine<L>::kFloats];
   // mirror pairs (t, TPL - t) in adjacent slots: lanes ^ TILE share W
   const int c = threadIdx.x % TILE, t = paired_slot_to_t(threadIdx.x / TILE, TPL);
-  const int row = blockIdx.x / NT;
-  int kjs[NL];
-  kjs[0] = JPAIR ? 1 + row : row * kj_step;
-  if constexpr (JPAIR) kjs[1] = L - 1 - row;
+  const int kj = blockIdx.x / NT;
   const int kp = (blockIdx.x % NT) * TILE + c;
   float* sre = lds + c * 2 * LdsLine<L>::kFloats;
   float* sim = sre + LdsLine<L>::kFloats;
-  float2 z[NL][E];
+  float2 z[E];
+  // element e of this line sits at line[e * L * L] (32-bit offsets: L^3 < 2^31)
+  const float2* __restrict__ src = spec + (long)kj * L + kp;
 #pragma unroll
-  for (int l = 0; l < NL; ++l) {
-    // element e of this line sits at line[e * L * L] (32-bit offsets: L^3 < 2^31)
-    const float2* __restrict__ src = spec + (long)kjs[l] * L + kp;
-#pragma unroll
-    for (int m = 0; m < E; ++m) z[l][m] = src[(t + TPL * m) * (L * L)];
-  }
-#pragma unroll
-  for (int l = 0; l < NL; ++l) line_fft<L, -1>(z[l], sre, sim, t, tw);
-  const int mjp = fold_sq(kjs[0], L) + fold_sq(kp, L);
+  for (int m = 0; m < E; ++m) z[m] = src[(t + TPL * m) * (L * L)];
+  line_fft<L, -1>(z, sre, sim, t, tw);
+  const int mjp = fold_sq(kj, L) + fold_sq(kp, L);
   // |k|^2 and its square root for the lower-half positions (radius-independent)
   int mm[E / 2 + 1];
   SqrtPair sq[E / 2 + 1];
@@ -299,20 +410,17 @@ __global__ __launch_bounds__(TILE*(L / Plan<L>::E)) void k_filter_i(
     } else {
       w_line_shared<L, E, TILE>(kappa[r], sq, mm, t, wv);  // dk R as hi + lo
     }
+    float2 v[E];
 #pragma unroll
-    for (int l = 0; l < NL; ++l) {
-      float2 v[E];
+    for (int m = 0; m < E; ++m) v[m] = make_float2(z[m].x * wv[m], z[m].y * wv[m]);
+    line_fft<L, +1>(v, sre, sim, tl, tw);
+    // t16: as k_filter_tab
+    float2* __restrict__ dst =
+        u + (long)r * ustride +
+        (t16 ? t16_tile<L>(0, kp >> 4) + kj * 16 + (kp & 15) : (long)kj * L + kp);
 #pragma unroll
-      for (int m = 0; m < E; ++m) v[m] = make_float2(z[l][m].x * wv[m], z[l][m].y * wv[m]);
-      line_fft<L, +1>(v, sre, sim, tl, tw);
-      // t16: the j pass's layout -- 16-column tiles of the (j, p) plane stored
-      // as contiguous L x 16 blocks, element (j, p) at (p/16) 16 L + 16 j + p%16
-      float2* __restrict__ dst =
-          u + (long)r * ustride +
-          (t16 ? (long)(kp >> 4) * (L * 16) + (long)kjs[l] * 16 + (kp & 15) : (long)kjs[l] * L + kp);
-#pragma unroll
-      for (int m = 0; m < E; ++m) st_stream(dst + (tl + TPL * m) * (L * L), v[m]);
-    }
+    for (int m = 0; m < E; ++m)
+      st_stream(dst + (t16 ? t16_tile<L>(tl + TPL * m, 0) : (long)(tl + TPL * m) * (L * L)), v[m]);
   }
 }
 
@@ -322,7 +430,11 @@ __global__ __launch_bounds__(TILE*(L / Plan<L>::E)) void k_filter_i(
 // among the batch's radii at which it is a centre.  Batches are issued in
 // ascending radius, so a batch's bounds exceed every earlier batch's and a
 // plain store (only where some centre was found) leaves in wmap the bound of
-// the largest radius -- no atomics and no reads of the map.  dbg (nullable)
+// the largest radius -- no atomics and no reads of the map.  A row's threads
+// sit in one wave, so the exchanges need no block barrier; the next radius is
+// loaded during the transform, and the twiddles stay in registers (a load of
+// them would wait for that prefetch).  Bound: HBM reads -- 512^3, 16 radii
+// 4.55 -> 2.62 ms per launch (6.4 TB/s), 256^3 0.42 -> 0.29 ms.  dbg (nullable)
 // receives the unscaled filtered pairs, keep (nullable) the pairs as
 // computed (N^3 rec_R, s N^3 ion_R), for the differentiable mode's backward.
 // ------------------------------------------------------------------------
@@ -336,47 +448,170 @@ __global__ __launch_bounds__(256) void k_inv_rows_crit(const float2* __restrict_
                                                        float2* __restrict__ keep,
                                                        const float2* __restrict__ tw, int t16) {
   constexpr int TPL = L / E, LPB = 256 / TPL;
+  static_assert(L % LPB == 0 && TPL % 16 == 0, "the block's rows in one plane, whole tiles");
   __shared__ float lds[LPB * 2 * LdsLine<L>::kFloats];
   const int lw = threadIdx.x / TPL, t = threadIdx.x % TPL;
-  const long row = (long)blockIdx.x * LPB + lw;
+  const int plane = blockIdx.x / (L / LPB);
+  const unsigned j = (blockIdx.x % (L / LPB)) * LPB + lw;  // row within the plane
+  const long row = (long)plane * L + j;
   float* sre = lds + lw * 2 * LdsLine<L>::kFloats;
   float* sim = sre + LdsLine<L>::kFloats;
   const float sc = bal[0];
+  // element p = t + TPL m of the row sits at voff plus a step in m of the plane:
+  // a per-thread offset plus a uniform one (scalar address arithmetic).
+  const unsigned voff = t16 ? 16 * j + (unsigned)t16_tile<L>(0, t >> 4) + (t & 15) : j * L + t;
   int wbest[E];
 #pragma unroll
   for (int m = 0; m < E; ++m) wbest[m] = -1;
+  float2 nx[E];
+  auto fetch = [&](int r) {
+    const float2* __restrict__ src =
+        vin + (long)r * vstride + (t16 ? t16_tile<L>(plane, 0) : (long)plane * (L * L));
+    if (t16) {
+#pragma unroll
+      for (int m = 0; m < E; ++m) nx[m] = ld_stream(uniform_ptr(src + m * TPL * L * L) + voff);
+    } else {
+#pragma unroll
+      for (int m = 0; m < E; ++m) nx[m] = ld_stream(uniform_ptr(src + TPL * m) + voff);
+    }
+  };
+  TwRegs<L, E> wr;
+  wr.load(t, tw);
+  fetch(nrad - 1);
+  // smallest radius first: the bounds grow along the walk, so the last
+  // centre found is the largest
 #pragma unroll 1
-  for (int r = 0; r < nrad; ++r) {
+  for (int r = nrad - 1; r >= 0; --r) {
     const int tl = opaque_lane(t);
     float2 v[E];
-    if (t16) {
-      // 16-column tile layout: element p of row (i, j) at i L^2 + (p/16) 16 L
-      // + 16 j + p%16
-      const float2* __restrict__ src =
-          vin + (long)r * vstride + (row / L) * ((long)L * L) + (row % L) * 16;
 #pragma unroll
-      for (int m = 0; m < E; ++m) {
-        const int p = tl + TPL * m;
-        v[m] = ld_stream(src + (p >> 4) * (L * 16) + (p & 15));
-      }
-    } else {
-      const float2* __restrict__ src = vin + (long)r * vstride + row * L;
-#pragma unroll
-      for (int m = 0; m < E; ++m) v[m] = ld_stream(src + tl + TPL * m);
-    }
-    line_fft_e<L, E, +1>(v, sre, sim, tl, tw);
+    for (int m = 0; m < E; ++m) v[m] = nx[m];
+    if (r > 0) fetch(r - 1);  // in flight during the transform
+    loop_fft<L, E, +1, true, true>(v, sre, sim, tl, wr);
     const int w = d2max[r];
+    // Re = N^3 rec_R, Im = s N^3 ion_R: centre test on (s rec_R, s ion_R)
 #pragma unroll
-    for (int m = 0; m < E; ++m) {
-      // Re = N^3 rec_R, Im = s N^3 ion_R: centre test on (s rec_R, s ion_R)
-      if (is_centre(v[m].x * sc, v[m].y)) wbest[m] = max(wbest[m], w);
-      if (dbg) dbg[(long)r * vstride + row * L + tl + TPL * m] = make_float2(v[m].x, v[m].y / sc);
-      if (keep) st_stream(keep + (long)r * vstride + row * L + tl + TPL * m, v[m]);
+    for (int m = 0; m < E; ++m) wbest[m] = is_centre(v[m].x * sc, v[m].y) ? w : wbest[m];
+    if (dbg) {
+#pragma unroll
+      for (int m = 0; m < E; ++m)
+        dbg[(long)r * vstride + row * L + tl + TPL * m] = make_float2(v[m].x, v[m].y / sc);
+    }
+    if (keep) {
+#pragma unroll
+      for (int m = 0; m < E; ++m) st_stream(keep + (long)r * vstride + row * L + tl + TPL * m, v[m]);
     }
   }
 #pragma unroll
   for (int m = 0; m < E; ++m)
     if (wbest[m] >= 0) wmap[row * L + t + TPL * m] = wbest[m];
+}
+
+// ------------------------------------------------------------------------
+// Sides up to 128: the inverse transforms along j and p and the centre test
+// of one (i, radius) plane in one block, the plane in registers (E values per
+// thread) and its exchanges in LDS: the filtered lines are read once and
+// nothing is written back between the two axes.  u in the natural layout, so
+// a plane is one contiguous read.  blockIdx.y: groups of rper radii (wmap by
+// atomic maximum when there are several).
+// Column phase: thread = column c, values j = tc + TPL m, as k_cols.  Row
+// phase: TPL threads per row in one wave, as k_inv_rows_crit; rows SR floats
+// apart (SR = 8 mod 32: the four rows of a half wave fall into disjoint banks).
+// Up to 128 a plane fits the 160 KiB of LDS and the registers of one block; at
+// 192 it no longer does.  Bound: LDS exchanges and VALU (one block per CU at
+// 128).  Against separate j and p passes, 16 radii: 128^3 0.124 -> 0.078 ms,
+// 64^3 (11 radii per launch, 128 blocks walking the radii) 0.049 -> 0.013 ms.
+// ------------------------------------------------------------------------
+template <int L>
+struct PlaneCfg {
+  static constexpr int E = L == 128 ? 16 : Plan<L>::E;
+  static constexpr int TPL = L / E;
+  static constexpr int kThreads = L * TPL;
+  static constexpr int SC = 2 * LdsLine<L>::kFloats;               // column regions
+  static constexpr int SR = SC + ((8 - SC % 32) + 32) % 32;        // row regions
+  static constexpr int kLds = (L * SR + 2 * L) * (int)sizeof(float);
+};
+
+template <int L>
+__global__ __launch_bounds__(PlaneCfg<L>::kThreads) void k_plane_crit(
+    const float2* __restrict__ u, int nrad, int rper, long ustride, const int* __restrict__ d2max,
+    const float* __restrict__ bal, int* __restrict__ wmap, float2* __restrict__ dbg,
+    float2* __restrict__ keep, const float2* __restrict__ tw) {
+  using C = PlaneCfg<L>;
+  constexpr int E = C::E, TPL = C::TPL;
+  extern __shared__ float pls[];
+  // the twiddles in LDS: loads from memory inside the radius loop would wait
+  // for the next plane's
+  float2* twl = reinterpret_cast<float2*>(pls + L * C::SR);
+  const int tid = threadIdx.x, plane = blockIdx.x;
+  for (int q = tid; q < L; q += C::kThreads) twl[q] = tw[q];
+  const int c = tid % 16 + 16 * (tid / (16 * TPL)), tc = (tid / 16) % TPL;
+  const int j = tid / TPL, t = tid % TPL;
+  float* cre = pls + c * C::SC;
+  float* cim = cre + LdsLine<L>::kFloats;
+  float* rre = pls + j * C::SR;
+  float* rim = rre + LdsLine<L>::kFloats;
+  const float sc = bal[0];
+  const long row = (long)plane * L + j;
+  const int r0 = blockIdx.y * rper, r1 = min(r0 + rper, nrad);
+  int wbest[E];
+#pragma unroll
+  for (int m = 0; m < E; ++m) wbest[m] = -1;
+  float2 nx[E];
+  const unsigned off = tc * L + c;
+  auto fetch = [&](int r) {
+    const float2* __restrict__ src = u + (long)r * ustride + (long)plane * (L * L);
+#pragma unroll
+    for (int m = 0; m < E; ++m) nx[m] = ld_stream(uniform_ptr(src + TPL * m * L) + off);
+  };
+  fetch(r1 - 1);
+  __syncthreads();
+  // smallest radius first: the last centre found has the largest bound
+#pragma unroll 1
+  for (int r = r1 - 1; r >= r0; --r) {
+    const int tcl = opaque_lane(tc), tl = opaque_lane(t);
+    float2 v[E];
+#pragma unroll
+    for (int m = 0; m < E; ++m) v[m] = nx[m];
+    loop_fft<L, E, +1>(v, cre, cim, tcl, twl);
+    if (r > r0) fetch(r - 1);  // in flight during the row phase
+    // to rows: element (j, p) at p of row region j
+#pragma unroll
+    for (int m = 0; m < E; ++m) {
+      float* o = pls + (tcl + TPL * m) * C::SR + lds_pad_u(c);
+      o[0] = v[m].x;
+      o[LdsLine<L>::kFloats] = v[m].y;
+    }
+    exchange_sync<false>();
+#pragma unroll
+    for (int m = 0; m < E; ++m) {
+      const unsigned o = lds_pad_u(tl + TPL * m);
+      v[m] = make_float2(rre[o], rim[o]);
+    }
+    exchange_sync<true>();
+    loop_fft<L, E, +1, true, true>(v, rre, rim, tl, twl);
+    const int w = d2max[r];
+    // Re = N^3 rec_R, Im = s N^3 ion_R: centre test on (s rec_R, s ion_R)
+#pragma unroll
+    for (int m = 0; m < E; ++m) wbest[m] = is_centre(v[m].x * sc, v[m].y) ? w : wbest[m];
+    if (dbg) {
+#pragma unroll
+      for (int m = 0; m < E; ++m)
+        dbg[(long)r * ustride + row * L + tl + TPL * m] = make_float2(v[m].x, v[m].y / sc);
+    }
+    if (keep) {
+#pragma unroll
+      for (int m = 0; m < E; ++m) st_stream(keep + (long)r * ustride + row * L + tl + TPL * m, v[m]);
+    }
+    exchange_sync<false>();  // the row regions are read before the next columns land in them
+  }
+#pragma unroll
+  for (int m = 0; m < E; ++m)
+    if (wbest[m] >= 0) {
+      int* w = wmap + row * L + t + TPL * m;
+      if (gridDim.y > 1) atomicMax(w, wbest[m]);
+      else *w = wbest[m];
+    }
 }
 
 __global__ void k_fill_i32(int* __restrict__ p, int value, long count) {
@@ -773,7 +1008,9 @@ static void cols_t(int width, int axis, int sign, const float2* in, float2* out,
 // buffers with width a multiple of the tile; the per-radius passes)
 void launch_cols(int n, int width, int axis, int sign, const float2* in, float2* out,
                  int nbatch, long bstride, const float2* tw, hipStream_t s, int tile, int variant) {
-  const bool wide = variant & 1, pipe = (variant & 2) != 0, nt = (variant & 4) != 0;
+  // forward transforms keep the size's own E: the compiler fuses other
+  // products in the wide forward butterflies, which moves last bits
+  const bool wide = (variant & 1) && sign > 0, pipe = (variant & 2) != 0, nt = (variant & 4) != 0;
   if ((variant & 8) && axis == 0 && width == n) axis = 2;  // the 16-column tile layout
 #define X(L)                                                                              \
   if (n == L) {                                                                           \
@@ -804,33 +1041,78 @@ void launch_cols(int n, int width, int axis, int sign, const float2* in, float2*
 #undef X
 }
 
+// Groups of radii per launch: enough that the blocks of one group times the
+// groups give the GPU about 16 waves per CU.
+static int radius_groups(long waves, int nrad) {
+  const long want = (4096 + waves - 1) / waves;
+  return (int)(want < 1 ? 1 : (want > nrad ? nrad : want));
+}
+
+void launch_w_table(int n, int nr, const float2* kappa, float* wt, hipStream_t s) {
+  hipLaunchKernelGGL(k_w_table, dim3((n + 15) / 16, n / 2 + 1, nr), dim3(256), 0, s, n, kappa, wt);
+}
+
 void launch_filter_i(int n, const float2* spec, float2* u, int nrad, long ustride,
-                     const float* wlut, long m_lut, const float2* kappa, const float2* tw,
-                     hipStream_t s, int tile, int wmode, bool jpair, bool t16) {
+                     const FilterW& w, int rb, const float2* tw, hipStream_t s, int tile, bool mirror,
+                     bool t16) {
   const int lay = t16 ? 1 : 0;
+  const float* wt = w.table ? w.table + rb * wtab_radius(n) : nullptr;
+  const float* lut = w.lut ? w.lut + (long)rb * w.mlut : nullptr;
 #define X(L, TL)                                                                          \
   if (n == L && tile == TL) {                                                             \
-    constexpr int NT = TL * (L / Plan<L>::E);                                             \
-    if (jpair && TL >= 8 && wmode != 0) {                                                 \
-      /* mirror pairs (kj, L - kj), kj = 1 .. L/2 - 1, then the lines 0 and L/2 */        \
-      const dim3 g((L / 2 - 1) * (L / TL)), g0(2 * (L / TL));                             \
-      hipLaunchKernelGGL((k_filter_i<L, TL, false, true>), g, dim3(NT), 0, s, spec, u,    \
-                         nrad, ustride, wlut, m_lut, kappa, tw, 0, lay);                  \
-      hipLaunchKernelGGL((k_filter_i<L, TL, false>), g0, dim3(NT), 0, s, spec, u, nrad,   \
-                         ustride, wlut, m_lut, kappa, tw, L / 2, lay);                    \
-      return;                                                                             \
+    constexpr int NT = TL * (L / Plan<L>::E), CT = L / TL;                                \
+    if (w.mode == 0)                                                                      \
+      hipLaunchKernelGGL((k_filter_i<L, TL, true>), dim3(L * CT), dim3(NT), 0, s, spec, u, nrad, \
+                         ustride, lut, w.mlut, w.kappa + rb, tw, lay);                    \
+    else if (!wt)                                                                         \
+      hipLaunchKernelGGL((k_filter_i<L, TL, false>), dim3(L * CT), dim3(NT), 0, s, spec, u, nrad, \
+                         ustride, lut, w.mlut, w.kappa + rb, tw, lay);                    \
+    else {                                                                                \
+      constexpr int NTF = TL * (L / FilterE<L>::kE);                                      \
+      const int g = radius_groups((long)L * CT * ((NTF + 63) / 64), nrad);                \
+      const int per = (nrad + g - 1) / g;                                                 \
+      const int mir = mirror && (L * CT) % 16 == 0;                                       \
+      hipLaunchKernelGGL((k_filter_tab<L, TL>), dim3(L * CT, (nrad + per - 1) / per), dim3(NTF), \
+                         0, s, spec, u, nrad, per, ustride, wt, tw, mir, lay);            \
     }                                                                                     \
-    if (wmode == 0)                                                                       \
-      hipLaunchKernelGGL((k_filter_i<L, TL, true>), dim3(L * (L / TL)), dim3(NT), 0, s, spec, u, \
-                         nrad, ustride, wlut, m_lut, kappa, tw, 1, lay);                  \
-    else                                                                                  \
-      hipLaunchKernelGGL((k_filter_i<L, TL, false>), dim3(L * (L / TL)), dim3(NT), 0, s, spec, u, \
-                         nrad, ustride, wlut, m_lut, kappa, tw, 1, lay);                  \
     return;                                                                               \
   }
 #define Y(L) X(L, 4) X(L, 8) X(L, 16)
   Y(32) Y(64) Y(96) Y(128) Y(192) Y(256) Y(512)
 #undef Y
+#undef X
+}
+
+bool plane_side(int n) { return n == 32 || n == 64 || n == 96 || n == 128; }
+
+#define SF21_PLANE_SIDES(X) X(32) X(64) X(96) X(128)
+
+bool plane_prepare(int n) {
+  // LDS above 64 KiB is requested per kernel
+  bool ok = true;
+#define X(L)                                                                              \
+  if (n == L)                                                                             \
+    ok = hipFuncSetAttribute((const void*)k_plane_crit<L>,                                \
+                             hipFuncAttributeMaxDynamicSharedMemorySize,                  \
+                             PlaneCfg<L>::kLds) == hipSuccess;
+  SF21_PLANE_SIDES(X)
+#undef X
+  return ok;
+}
+
+void launch_plane_crit(int n, const float2* u, int nrad, long ustride, const int* d2max,
+                       const float* bal, int* wmap, float2* dbg, float2* keep, const float2* tw,
+                       hipStream_t s) {
+#define X(L)                                                                              \
+  if (n == L) {                                                                           \
+    const int g = radius_groups((long)L * ((PlaneCfg<L>::kThreads + 63) / 64), nrad);     \
+    const int per = (nrad + g - 1) / g;                                                   \
+    hipLaunchKernelGGL(k_plane_crit<L>, dim3(L, (nrad + per - 1) / per),                  \
+                       dim3(PlaneCfg<L>::kThreads), PlaneCfg<L>::kLds, s, u, \
+                       nrad, per, ustride, d2max, bal, wmap, dbg, keep, tw);              \
+    return;                                                                               \
+  }
+  SF21_PLANE_SIDES(X)
 #undef X
 }
 
@@ -852,8 +1134,8 @@ void launch_inv_rows_crit(int n, const float2* v, int nrad, long vstride, const 
                        d2max, bal, wmap, dbg, keep, tw, lay);                                   \
     return;                                                                               \
   }
-  XW(128) XW(256) XW(512)
-  SF21_SIZES(X)
+  XW(256) XW(512)
+  X(192) X(256) X(512)
 #undef XW
 #undef X
 }

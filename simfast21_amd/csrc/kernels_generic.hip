@@ -187,7 +187,7 @@ __device__ __forceinline__ void gen_last(const GenPlan& P, int st, int jj, const
       a[r] = line[T1 ? gen_t1_slot(o, L >> 3) : o];
     }
     gen_twiddle<R, SIGN>(a, j, tstep, tw);
-    Dft<R, SIGN>::run(a);
+    Dft<R, SIGN, MODE == 2>::run(a);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const unsigned idx = base + (unsigned)(j + r * Lr) * stride;

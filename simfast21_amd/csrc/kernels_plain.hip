@@ -33,15 +33,14 @@ __global__ __launch_bounds__(256) void k_r2c_rows(const float* __restrict__ in,
   float2 v[E];
 #pragma unroll
   for (int m = 0; m < E; ++m) v[m] = rin[t + TPL * m];
-  line_fft<H, -1>(v, sre, sim, t, twh);
+  line_fft<H, -1, true>(v, sre, sim, t, twh);
 #pragma unroll
   for (int m = 0; m < E; ++m) {
     const int o = lds_pad(t + TPL * m);
     sre[o] = v[m].x;
     sim[o] = v[m].y;
   }
-  lds_pin();
-  __syncthreads();
+  exchange_sync<true>();
   float2* __restrict__ rout = out + row * (H + 1);
 #pragma unroll
   for (int m = 0; m < E; ++m) {
@@ -89,7 +88,7 @@ __global__ __launch_bounds__(256) void k_c2r_rows(const float2* __restrict__ in,
     const float tr = w.x * dr + w.y * di, ti = w.x * di - w.y * dr;
     v[m] = make_float2(sr - ti, si + tr);
   }
-  line_fft<H, +1>(v, sre, sim, t, twh);
+  line_fft<H, +1, true>(v, sre, sim, t, twh);
   float2* __restrict__ rout = reinterpret_cast<float2*>(out + row * L);
 #pragma unroll
   for (int m = 0; m < E; ++m) rout[t + TPL * m] = v[m];
@@ -107,7 +106,7 @@ __global__ __launch_bounds__(256) void k_c2c_rows(float2* __restrict__ data,
   float2 v[E];
 #pragma unroll
   for (int m = 0; m < E; ++m) v[m] = data[row * L + t + TPL * m];
-  line_fft<L, SIGN>(v, sre, sim, t, tw);
+  line_fft<L, SIGN, true>(v, sre, sim, t, tw);
 #pragma unroll
   for (int m = 0; m < E; ++m) data[row * L + t + TPL * m] = v[m];
 }

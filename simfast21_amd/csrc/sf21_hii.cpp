@@ -106,6 +106,10 @@ struct sf21_hii_ctx {
   std::vector<double> radii;
   std::vector<int> d2;
   int n = 0, h = 0, K = 0;
+  // radii per batch of the differentiable backward (K, or 16 where K is the
+  // automatic whole ladder): its accumulators are summed batch by batch, so the
+  // grouping is part of the gradient's last bits
+  int Kd = 0;
   int tile_filter = 16;
   int cols_tile = 16;  // columns per block of the per-radius passes along j
   int cols_wide = 0;  // per-radius passes along j: bit 0 16 values per thread, bit 1 prefetching blocks
@@ -124,6 +128,8 @@ struct sf21_hii_ctx {
   float2 *tw = nullptr, *twh = nullptr;
   float* wlut = nullptr;
   long mlut = 0;
+  float* wtab = nullptr;  // FP32 top-hat weights per radius (wtab_radius floats each)
+  bool plane = false;     // j and p inverses and centre test plane by plane
   int* d_d2 = nullptr;
   // fused path
   float2 *spec = nullptr, *ubuf = nullptr;
@@ -344,6 +350,10 @@ void enqueue_generic(sf21_hii_ctx* c, const float* a, const float* b, const floa
   });
 }
 
+FilterW filter_weights(const sf21_hii_ctx* c) {
+  return FilterW{c->filter_w, c->wlut, c->mlut, c->wtab, c->d_kappa};
+}
+
 // ---- fused exact path: enqueue one slice -------------------------------
 // keep (nullable): the filtered pairs of every radius, radius r at keep + r n^3
 void enqueue_fused(sf21_hii_ctx* c, const float* a, const float* b, const float* cc, double z,
@@ -370,10 +380,16 @@ void enqueue_fused(sf21_hii_ctx* c, const float* a, const float* b, const float*
     const int rb = std::max(r_lo, re - c->K);
     const int kk = re - rb;
     launch(c, "filter_i", [&] {
-      launch_filter_i(n, c->spec, c->ubuf, kk, n3, c->wlut + (long)rb * c->mlut, c->mlut,
-                      c->d_kappa + rb, c->tw, s, c->tile_filter, c->filter_w, c->filter_pair,
-                      true);
+      launch_filter_i(n, c->spec, c->ubuf, kk, n3, filter_weights(c), rb, c->tw, s, c->tile_filter,
+                      c->filter_pair, !c->plane);
     });
+    if (c->plane) {
+      launch(c, "plane_crit", [&] {
+        launch_plane_crit(n, c->ubuf, kk, n3, c->d_d2 + rb, c->bal, c->wmap, dbg,
+                          keep ? keep + (long)rb * n3 : nullptr, c->tw, s);
+      });
+      continue;
+    }
     launch(c, "cols_inv_j", [&] {
       launch_cols(n, n, 0, +1, c->ubuf, c->ubuf, kk, n3, c->tw, s, c->cols_tile,
                   c->cols_wide | kColsStream | kColsT16);
@@ -473,7 +489,7 @@ void free_all(sf21_hii_ctx* c) {
   for (auto& g : c->graphs)
     if (g.exec) (void)hipGraphExecDestroy(g.exec);
   c->graphs.clear();
-  dev_free(c->tw); dev_free(c->twh); dev_free(c->wlut); dev_free(c->d_d2); dev_free(c->d_kappa);
+  dev_free(c->tw); dev_free(c->twh); dev_free(c->wlut); dev_free(c->wtab); dev_free(c->d_d2); dev_free(c->d_kappa);
   dev_free(c->spec); dev_free(c->ubuf); dev_free(c->wmap); dev_free(c->gbuf);
   dev_free(c->bal_part); dev_free(c->bal); dev_free(c->partials); dev_free(c->neutral_dev);
   dev_free(c->rec); dev_free(c->ion); dev_free(c->fres); dev_free(c->bubblef);
@@ -578,7 +594,7 @@ int ensure_diff(sf21_hii_ctx* c) {
   if (c->df_ready) return SF21_OK;
   const size_t n3 = (size_t)c->n3, nh = (size_t)c->nh;
   const size_t h = (size_t)(c->n / 2 + 1);
-  const size_t npair = (size_t)(c->K + 1) / 2;
+  const size_t npair = (size_t)(c->Kd + 1) / 2;
   int rc;
   if ((rc = dev_alloc(&c->df_delta, n3)) || (rc = dev_alloc(&c->df_rec, n3)) ||
       (rc = dev_alloc(&c->df_ion, n3)) || (rc = dev_alloc(&c->df_x, n3)) ||
@@ -669,8 +685,8 @@ void enqueue_diff_backward(sf21_hii_ctx* c, const float* g, const float* emis, d
   }
   // sweep 1: C = sum_R B_R FFT(phi_R)
   launch(c, "diff_fill", [&] { launch_fill_c(c->df_c, n3, s); });
-  for (int rb = 0; rb < nr; rb += c->K) {
-    const int kk = std::min(c->K, nr - rb);
+  for (int rb = 0; rb < nr; rb += c->Kd) {
+    const int kk = std::min(c->Kd, nr - rb);
     const int kp = (kk + 1) / 2;
     if (kept) {
       launch(c, "rows_phi", [&] {
@@ -679,8 +695,8 @@ void enqueue_diff_backward(sf21_hii_ctx* c, const float* g, const float* emis, d
       });
     } else {
       launch(c, "filter_i", [&] {
-        launch_filter_i(n, c->spec, c->ubuf, kk, n3, c->wlut + (long)rb * c->mlut, c->mlut,
-                        c->d_kappa + rb, c->tw, s, c->tile_filter, c->filter_w, c->filter_pair);
+        launch_filter_i(n, c->spec, c->ubuf, kk, n3, filter_weights(c), rb, c->tw, s, c->tile_filter,
+                        c->filter_pair);
       });
       launch(c, "cols_inv_j", [&] { launch_cols(n, n, 0, +1, c->ubuf, c->ubuf, kk, n3, c->tw, s, c->cols_tile, c->cols_wide | kColsStream); });
       launch(c, "rows_phi", [&] {
@@ -719,8 +735,8 @@ void enqueue_diff_backward(sf21_hii_ctx* c, const float* g, const float* emis, d
     launch_fill_c(c->df_g, n3, s);
     launch_fill_d(c->df_rho, rows_blocks(n), s);
   });
-  for (int rb = 0; rb < nr; rb += c->K) {
-    const int kk = std::min(c->K, nr - rb);
+  for (int rb = 0; rb < nr; rb += c->Kd) {
+    const int kk = std::min(c->Kd, nr - rb);
     const int kp = (kk + 1) / 2;
     launch(c, "ball_i", [&] {
       launch_ball_i(n, false, c->df_c, 0, c->df_v, n3, kk, c->df_ball + (long)rb * h3, c->tw, s);
@@ -728,8 +744,8 @@ void enqueue_diff_backward(sf21_hii_ctx* c, const float* g, const float* emis, d
     launch(c, "cols_inv_j", [&] { launch_cols(n, n, 0, +1, c->df_v, c->df_v, kp, n3, c->tw, s, c->cols_tile, c->cols_wide | kColsStream); });
     if (!c->df_pairs) {  // recompute the batch's filtered pairs
       launch(c, "filter_i", [&] {
-        launch_filter_i(n, c->spec, c->ubuf, kk, n3, c->wlut + (long)rb * c->mlut, c->mlut,
-                        c->d_kappa + rb, c->tw, s, c->tile_filter, c->filter_w, c->filter_pair);
+        launch_filter_i(n, c->spec, c->ubuf, kk, n3, filter_weights(c), rb, c->tw, s, c->tile_filter,
+                        c->filter_pair);
       });
       launch(c, "cols_inv_j", [&] { launch_cols(n, n, 0, +1, c->ubuf, c->ubuf, kk, n3, c->tw, s, c->cols_tile, c->cols_wide | kColsStream); });
     }
@@ -739,7 +755,7 @@ void enqueue_diff_backward(sf21_hii_ctx* c, const float* g, const float* emis, d
     });
     launch(c, "cols_fwd_j", [&] { launch_cols(n, n, 0, -1, c->ubuf, c->ubuf, kk, n3, c->tw, s, c->cols_tile, c->cols_wide | kColsStream); });
     launch(c, "filter_acc_i", [&] {
-      launch_filter_acc_i(n, c->ubuf, n3, kk, c->wlut + (long)rb * c->mlut, c->mlut, c->d_kappa + rb,
+      launch_filter_acc_i(n, c->ubuf, n3, kk, c->wlut ? c->wlut + (long)rb * c->mlut : nullptr, c->mlut, c->d_kappa + rb,
                           c->filter_w, c->df_g, c->tw, s);
     });
   }
@@ -978,7 +994,7 @@ void drop_graphs(sf21_hii_ctx* c) {
 int set_radius_batch(sf21_hii_ctx* c, int K) {
   if (K > (int)c->radii.size()) K = (int)c->radii.size();
   if (K < 1) return SF21_ERR_ARG;
-  if (K == c->K) return SF21_OK;
+  if (K == c->K && K == c->Kd) return SF21_OK;
   if (hipStreamSynchronize(c->stream) != hipSuccess) return SF21_ERR_HIP;
   drop_graphs(c);
   dev_free(c->ubuf);
@@ -988,10 +1004,10 @@ int set_radius_batch(sf21_hii_ctx* c, int K) {
     if (dev_alloc(&c->ubuf, (size_t)c->n3 * c->K)) return SF21_ERR_ALLOC;
     return rc;
   }
-  c->K = K;
+  c->K = c->Kd = K;
   if (c->df_v) {
     dev_free(c->df_v);
-    if ((rc = dev_alloc(&c->df_v, (size_t)(c->K + 1) / 2 * c->n3))) {
+    if ((rc = dev_alloc(&c->df_v, (size_t)(c->Kd + 1) / 2 * c->n3))) {
       c->df_ready = false;
       return rc;
     }
@@ -1181,6 +1197,7 @@ int sf21_hii_create(const sf21_hii_config* cfg, sf21_hii_ctx** out) {
   c->filter_w = cfg->filter_w == 2 ? 0 : 1;
   // untuned: mirror-paired filter blocks where the pairs still fill the GPU
   c->filter_pair = c->n >= 256 && c->tile_filter >= 8 && c->filter_w;
+  c->cols_wide = c->n >= 256 ? cols_variant(c->n, c->cols_tile, 1) : 0;
   if (tuned) {
     c->tile_filter = tc.tile;
     c->cols_tile = tc.ct;
@@ -1188,10 +1205,30 @@ int sf21_hii_create(const sf21_hii_config* cfg, sf21_hii_ctx** out) {
     c->rows_wide = tc.rw && wide_ok(c->n);
     c->filter_pair = tc.fp && tc.tile >= 8 && c->filter_w;
   }
+  if (cfg->path == SF21_PATH_FUSED && !c->generic && cfg->radius_batch <= 0 && !tuned) {
+    // automatic batch: the whole ladder (the spectrum is read and transformed
+    // along i once per batch: at 512^3 and 47 radii 11.2 ms of filter passes
+    // per slice against 13.1 ms in batches of 16) while its pairs take at most
+    // a third of the free memory, else halved down to 16
+    size_t free_b = 0, total_b = 0;
+    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = 0;
+    (void)hipGetLastError();
+    c->K = (int)c->radii.size();
+    while (c->K > 16 && sizeof(float2) * (size_t)c->n3 * c->K > free_b / 3) c->K = (c->K + 1) / 2;
+    if (c->K < 16) c->K = 16;
+    c->Kd = 16;
+  }
   if (c->K > (int)c->radii.size()) c->K = (int)c->radii.size();
   if (c->generic) c->K = 1;  // one radius per step, in-kernel FP32 weights
   if (c->generic) c->filter_w = 1;
+  if (c->Kd < 1 || c->Kd > c->K) c->Kd = c->K;
 
+  c->plane = !c->generic && plane_side(c->n);
+  if (c->plane && !plane_prepare(c->n)) {
+    (void)hipGetLastError();
+    delete c;
+    return SF21_ERR_HIP;
+  }
   if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) {
     delete c;
     return SF21_ERR_HIP;
@@ -1202,14 +1239,17 @@ int sf21_hii_create(const sf21_hii_config* cfg, sf21_hii_ctx** out) {
   {
     const int hh = c->n / 2;
     c->mlut = 3L * hh * hh + 1;
-    std::vector<float> w((size_t)c->mlut * c->radii.size());
-    for (size_t r = 0; r < c->radii.size(); ++r)
-      for (long m = 0; m < c->mlut; ++m)
-        w[r * c->mlut + m] = (float)w_filter(c->dk * std::sqrt((double)m) * c->radii[r]);
-    if ((rc = dev_alloc(&c->wlut, w.size()))) goto fail;
-    if (hipMemcpy(c->wlut, w.data(), sizeof(float) * w.size(), hipMemcpyHostToDevice) != hipSuccess) {
-      rc = SF21_ERR_HIP;
-      goto fail;
+    if (cfg->path == SF21_PATH_PLAIN || !c->filter_w) {  // the FP64 weight table per |k|^2
+      std::vector<float> w((size_t)c->mlut * c->radii.size());
+      for (size_t r = 0; r < c->radii.size(); ++r)
+        for (long m = 0; m < c->mlut; ++m)
+          w[r * c->mlut + m] = (float)w_filter(c->dk * std::sqrt((double)m) * c->radii[r]);
+      if ((rc = dev_alloc(&c->wlut, w.size()))) goto fail;
+      if (hipMemcpy(c->wlut, w.data(), sizeof(float) * w.size(), hipMemcpyHostToDevice) !=
+          hipSuccess) {
+        rc = SF21_ERR_HIP;
+        goto fail;
+      }
     }
     std::vector<float2> kap(c->radii.size());
     for (size_t r = 0; r < c->radii.size(); ++r) {
@@ -1223,6 +1263,17 @@ int sf21_hii_create(const sf21_hii_config* cfg, sf21_hii_ctx** out) {
         hipSuccess) {
       rc = SF21_ERR_HIP;
       goto fail;
+    }
+    if (c->filter_w && !c->generic) {
+      // the FP32 weight table, if it takes at most 1/16 of
+      // the free memory (otherwise the filter pass evaluates the weights)
+      const size_t count = (size_t)wtab_radius(c->n) * c->radii.size();
+      size_t free_b = 0, total_b = 0;
+      if (hipMemGetInfo(&free_b, &total_b) == hipSuccess && sizeof(float) * count <= free_b / 16 &&
+          dev_alloc(&c->wtab, count) == SF21_OK)
+        launch_w_table(c->n, (int)c->radii.size(), c->d_kappa, c->wtab, c->stream);
+      else
+        (void)hipGetLastError();
     }
     if ((rc = dev_alloc(&c->d_d2, c->d2.size()))) goto fail;
     if (hipMemcpy(c->d_d2, c->d2.data(), sizeof(int) * c->d2.size(), hipMemcpyHostToDevice) !=
@@ -1255,6 +1306,7 @@ int sf21_hii_create(const sf21_hii_config* cfg, sf21_hii_ctx** out) {
     while ((rc = dev_alloc(&c->ubuf, (size_t)c->n3 * c->K)) && cfg->radius_batch <= 0 && c->K > 1)
       c->K /= 2;
     if (rc) goto fail;
+    if (c->Kd > c->K) c->Kd = c->K;
     if ((rc = dev_alloc(&c->wmap, (size_t)c->n3)) || (rc = dev_alloc(&c->gbuf, (size_t)c->n3)) ||
         (rc = dev_alloc(&c->bal_part, (size_t)2 * balance_partials_count(c->n3))) ||
         (rc = dev_alloc(&c->bal, 1)) ||
@@ -1269,6 +1321,11 @@ int sf21_hii_create(const sf21_hii_config* cfg, sf21_hii_ctx** out) {
         (rc = dev_alloc(&c->tmp2, (size_t)(2 * c->nh))) || (rc = dev_alloc(&c->th, (size_t)c->nh)) ||
         (rc = dev_alloc(&c->flag_dev, 1)))
       goto fail;
+  }
+  // the tables are complete before any other stream can use them
+  if (hipStreamSynchronize(c->stream) != hipSuccess || (rc = check_hip())) {
+    if (!rc) rc = SF21_ERR_HIP;
+    goto fail;
   }
   *out = c;
   return SF21_OK;
@@ -1670,7 +1727,7 @@ int sf21_hii_autotune(sf21_hii_ctx* c, const float* a, const float* b, const flo
     t.fp = 1 - t.fp;
     consider(t);
   }
-  {
+  if (!c->plane) {  // plane sides have neither a j pass nor a p pass
     const TuneChoice base = best;
     const int cols_opts[7][2] = {{8, 0}, {16, 0}, {16, 2}, {16, 1}, {16, 3}, {32, 1}, {32, 3}};
     for (auto& o : cols_opts) {
@@ -1681,7 +1738,7 @@ int sf21_hii_autotune(sf21_hii_ctx* c, const float* a, const float* b, const flo
       if (t.ct != base.ct || t.cw != base.cw) consider(t);
     }
   }
-  if (wide_ok(c->n)) {
+  if (!c->plane && wide_ok(c->n)) {
     TuneChoice t = best;
     t.rw = 1;
     consider(t);
