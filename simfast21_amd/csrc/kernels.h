@@ -137,7 +137,11 @@ void launch_clamp_sum(long n3, float* bubblef, const float* fresid, double* part
 // ---- binned power spectrum ----
 int pk_partials_count(int n);
 // full: spec is the n^3 spectrum of a complex transform (its p <= n/2 half binned)
-void launch_power_spectrum(int n, const float2* spec, const short* bin_of_m, const float* kabs_of_m,
+// geo: sums of |k| per bin, then mode counts (depend on n and the bins only);
+// part: 2 nbins pk_partials_count(n) doubles
+void launch_pk_geometry(int n, const short* bin_of_m, const float* kabs_of_m, int nbins,
+                        double* part, double* geo, hipStream_t s);
+void launch_power_spectrum(int n, const float2* spec, const short* bin_of_m, const double* geo,
                            int nbins, double norm, double* part, double* out, hipStream_t s,
                            bool full = false);
 

@@ -152,6 +152,7 @@ struct sf21_hii_ctx {
   short* pk_bin = nullptr;
   float* pk_kabs = nullptr;
   double* pk_part = nullptr;
+  double* pk_geo = nullptr;  // per bin: sum of |k|, then mode count
   double* pk_out = nullptr;
   int pk_nbins = 0;
   // differentiable mode (allocated on first use)
@@ -497,7 +498,7 @@ void free_all(sf21_hii_ctx* c) {
   dev_free(c->spec2); dev_free(c->tmp2); dev_free(c->th); dev_free(c->flag_dev);
   dev_free(c->halo_grid); dev_free(c->halo_buf);
   dev_free(c->t21_dv); dev_free(c->t21_part); dev_free(c->sum_part);
-  dev_free(c->pk_bin); dev_free(c->pk_kabs); dev_free(c->pk_part); dev_free(c->pk_out);
+  dev_free(c->pk_bin); dev_free(c->pk_kabs); dev_free(c->pk_part); dev_free(c->pk_geo); dev_free(c->pk_out);
   dev_free(c->df_delta); dev_free(c->df_rec); dev_free(c->df_ion); dev_free(c->df_x);
   dev_free(c->df_t); dev_free(c->df_fq); dev_free(c->df_fa); dev_free(c->df_qbar);
   dev_free(c->df_dbar); dev_free(c->df_dd); dev_free(c->df_v); dev_free(c->df_c);
@@ -542,15 +543,17 @@ int ensure_pk(sf21_hii_ctx* c, int nbins) {
     kab[m] = (float)(kq * c->dk);
   }
   int rc;
-  dev_free(c->pk_bin); dev_free(c->pk_kabs); dev_free(c->pk_part); dev_free(c->pk_out);
+  dev_free(c->pk_bin); dev_free(c->pk_kabs); dev_free(c->pk_part); dev_free(c->pk_geo); dev_free(c->pk_out);
   c->pk_nbins = 0;
   if ((rc = dev_alloc(&c->pk_bin, bins.size())) || (rc = dev_alloc(&c->pk_kabs, kab.size())) ||
-      (rc = dev_alloc(&c->pk_part, (size_t)3 * nbins * pk_partials_count(c->n))) ||
+      (rc = dev_alloc(&c->pk_part, (size_t)2 * nbins * pk_partials_count(c->n))) ||
+      (rc = dev_alloc(&c->pk_geo, (size_t)2 * nbins)) ||
       (rc = dev_alloc(&c->pk_out, (size_t)3 * nbins)))
     return rc;
   if (hipMemcpy(c->pk_bin, bins.data(), sizeof(short) * bins.size(), hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(c->pk_kabs, kab.data(), sizeof(float) * kab.size(), hipMemcpyHostToDevice) != hipSuccess)
     return SF21_ERR_HIP;
+  launch_pk_geometry(c->n, c->pk_bin, c->pk_kabs, nbins, c->pk_part, c->pk_geo, c->stream);
   c->pk_nbins = nbins;
   return SF21_OK;
 }
@@ -574,7 +577,7 @@ void enqueue_pk(sf21_hii_ctx* c, const float* field, float2* half, int nbins) {
   const double dl = c->dx;
   const double norm = dl * dl * dl / ((double)c->n3);
   launch(c, "power_spectrum", [&] {
-    launch_power_spectrum(c->n, half, c->pk_bin, c->pk_kabs, nbins, norm, c->pk_part, c->pk_out,
+    launch_power_spectrum(c->n, half, c->pk_bin, c->pk_geo, nbins, norm, c->pk_part, c->pk_out,
                           s, c->generic);
   });
 }
