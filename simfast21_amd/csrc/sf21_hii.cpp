@@ -8,7 +8,6 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
-#include <mutex>
 #include <string>
 #include <vector>
 
@@ -178,7 +177,8 @@ struct sf21_hii_ctx {
   float* t21_dv = nullptr;      // velocity gradient (unnormalised C2R output)
   double* t21_part = nullptr;   // partial sums, then the two totals at the end
   // halo mode
-  float* halo_grid = nullptr;   // N_halo^3 deposit grid
+  float* halo_grid = nullptr;   // N_halo^3 grid of a density deposit that the caller does not take
+  double* halo_acc = nullptr;   // n^3 sums of a catalog deposit
   float* halo_buf = nullptr;    // catalog upload (host entry point)
   double* sum_part = nullptr;   // FP64 partial sums of a box, then the total
   long halo_cap = 0;
@@ -496,7 +496,7 @@ void free_all(sf21_hii_ctx* c) {
   dev_free(c->rec); dev_free(c->ion); dev_free(c->fres); dev_free(c->bubblef);
   dev_free(c->box_a); dev_free(c->box_b); dev_free(c->bubble);
   dev_free(c->spec2); dev_free(c->tmp2); dev_free(c->th); dev_free(c->flag_dev);
-  dev_free(c->halo_grid); dev_free(c->halo_buf);
+  dev_free(c->halo_grid); dev_free(c->halo_acc); dev_free(c->halo_buf);
   dev_free(c->t21_dv); dev_free(c->t21_part); dev_free(c->sum_part);
   dev_free(c->pk_bin); dev_free(c->pk_kabs); dev_free(c->pk_part); dev_free(c->pk_geo); dev_free(c->pk_out);
   dev_free(c->df_delta); dev_free(c->df_rec); dev_free(c->df_ion); dev_free(c->df_x);
@@ -1040,6 +1040,20 @@ void apply_choice(sf21_hii_ctx* c, const TuneChoice& t) {
   drop_graphs(c);
 }
 
+// Largest N_halo^3 that sf21_hii_halo_emissivity_noalloc takes (N_halo <= 256).
+constexpr long kNoAllocGrid = 1L << 24;
+
+// FP64 sums of the catalog deposits; left null (FP32 sums in the output box)
+// where they do not fit.  Contexts that sf21_hii_halo_emissivity_noalloc takes
+// allocate them when they are created.
+void ensure_halo_acc(sf21_hii_ctx* c) {
+  if (!c->halo_acc) (void)dev_alloc(&c->halo_acc, (size_t)c->n3);
+}
+bool noalloc_context(const sf21_hii_ctx* c) {
+  const long ng = c->cfg.n_halo;
+  return c->cfg.input_mode == SF21_INPUT_HALO && ng * ng * ng <= kNoAllocGrid;
+}
+
 // Deposit-only context: the stream and the parameters the deposit entry
 // points read; halo grid and sums are allocated on first use.
 int create_deposit(const sf21_hii_config* cfg, sf21_hii_ctx** out) {
@@ -1067,6 +1081,7 @@ int create_deposit(const sf21_hii_config* cfg, sf21_hii_ctx** out) {
     return SF21_ERR_HIP;
   }
   c->own_stream = true;
+  if (noalloc_context(c)) ensure_halo_acc(c);
   *out = c;
   return SF21_OK;
 }
@@ -1325,6 +1340,7 @@ int sf21_hii_create(const sf21_hii_config* cfg, sf21_hii_ctx** out) {
         (rc = dev_alloc(&c->flag_dev, 1)))
       goto fail;
   }
+  if (noalloc_context(c)) ensure_halo_acc(c);
   // the tables are complete before any other stream can use them
   if (hipStreamSynchronize(c->stream) != hipSuccess || (rc = check_hip())) {
     if (!rc) rc = SF21_ERR_HIP;
@@ -1832,18 +1848,6 @@ int sf21_hii_power_spectrum_dev(sf21_hii_ctx* c, const float* field, int nbins, 
 // ---- halo-catalog emissivity (get_HIIbubbles.c:229-259) -----------------
 }  // extern "C"
 
-// Scratch of sf21_hii_halo_emissivity_noalloc: the N_halo^3 CIC deposit
-// grid, at most kNoAllocGrid floats (64 MiB: N_halo <= 256), in a
-// file-scope device array that every GPU the library runs on holds from
-// module load until the process ends.  In host code the array's name is a
-// host-side stand-in, not a device address: each device's address comes
-// from hipGetSymbolAddress, taken once per device (with that device
-// current) on the entry point's first call there, and only that address is
-// passed to kernels.  Calls on one GPU share its array: each call zeroes the
-// grid before depositing, and calls that overlap on one GPU race.
-constexpr long kNoAllocGrid = 1L << 24;
-static __device__ __align__(256) float scratch[kNoAllocGrid];
-
 namespace {
 // Launch constants of the halo-mode emissivity: smooth_box's block size
 // (auxiliary.c:654-656), the volume ratio times fesc (get_HIIbubbles.c:253-258)
@@ -1863,26 +1867,6 @@ int halo_consts(const sf21_hii_ctx* c, double z, HaloConsts* k) {
   return SF21_OK;
 }
 
-constexpr int kMaxDevices = 64;
-std::mutex g_scratch_mu;
-float* g_scratch_dev[kMaxDevices] = {};
-
-// The device address of this device's scratch array (the device must be
-// current).
-int scratch_address(int device, float** out) {
-  if (device < 0 || device >= kMaxDevices) return SF21_ERR_ARG;
-  std::lock_guard<std::mutex> lock(g_scratch_mu);
-  if (!g_scratch_dev[device]) {
-    void* p = nullptr;
-    if (hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)) != hipSuccess || !p) {
-      (void)hipGetLastError();
-      return SF21_ERR_HIP;
-    }
-    g_scratch_dev[device] = static_cast<float*>(p);
-  }
-  *out = g_scratch_dev[device];
-  return SF21_OK;
-}
 }  // namespace
 
 extern "C" {
@@ -1895,14 +1879,10 @@ int sf21_hii_halo_emissivity_dev(sf21_hii_ctx* c, const float* halos, long nhalo
   if (halo_consts(c, z, &k)) return SF21_ERR_ARG;
   if (hipSetDevice(c->cfg.device) != hipSuccess) return SF21_ERR_HIP;
   (void)hipGetLastError();
-  const int ng = c->cfg.n_halo, ns = c->n;
-  if (!c->halo_grid) {
-    int rc = dev_alloc(&c->halo_grid, (size_t)ng * ng * ng);
-    if (rc) return rc;
-  }
+  ensure_halo_acc(c);
   launch(c, "halo_emissivity", [&] {
-    launch_halo_emissivity(nhalos, halos, ng, ns, (int)k.sm, k.k_rion, (float)9.367608e+07, 0.44f,
-                           k.scale, c->halo_grid, ion_out, c->stream);
+    launch_halo_emissivity(nhalos, halos, c->cfg.n_halo, c->n, (int)k.sm, k.k_rion,
+                           (float)9.367608e+07, 0.44f, k.scale, c->halo_acc, ion_out, c->stream);
   });
   if (hipStreamSynchronize(c->stream) != hipSuccess) return SF21_ERR_HIP;
   if (c->prof) collect(c);
@@ -1919,12 +1899,9 @@ int sf21_hii_halo_emissivity_noalloc(sf21_hii_ctx* c, const float* halos, long n
   if (halo_consts(c, z, &k)) return SF21_ERR_ARG;
   if (hipSetDevice(c->cfg.device) != hipSuccess) return SF21_ERR_HIP;
   (void)hipGetLastError();
-  float* grid = nullptr;
-  int rc = scratch_address(c->cfg.device, &grid);
-  if (rc) return rc;
   // enqueued on the context's stream, no host synchronisation (capturable)
   launch_halo_emissivity(nhalos, halos, (int)ng, c->n, (int)k.sm, k.k_rion, (float)9.367608e+07,
-                         0.44f, k.scale, grid, ion_out, c->stream);
+                         0.44f, k.scale, c->halo_acc, ion_out, c->stream);
   return check_hip();
 }
 
@@ -2057,17 +2034,17 @@ int sf21_sfrd_dev(sf21_hii_ctx* c, const float* halos, long nhalos, double z, fl
   if (hipSetDevice(c->cfg.device) != hipSuccess) return SF21_ERR_HIP;
   (void)hipGetLastError();
   int rc;
-  if ((rc = ensure_halo_grid(c))) return rc;
   const int ng = c->cfg.n_halo, ns = c->n;
   const long sm = smooth_block(ng, ns);
   if (sm < 1) return SF21_ERR_ARG;
+  ensure_halo_acc(c);
   const double dx_h = c->L / ng;
   // sfr = Rion/Qion (user_functions.c:71-74); Msun/yr per halo, then the
   // block average divided by dx_halo^3 (get_SFR.c:126-139)
   const float k_sfr = (float)(1.575e39 * std::pow(1.0 + z, 2.27044695e+00) / kVnorm / fit_Qion(z));
   launch(c, "sfrd", [&] {
     launch_halo_emissivity(nhalos, halos, ng, ns, (int)sm, k_sfr, (float)9.367608e+07, 0.44f,
-                           (float)(1.0 / (dx_h * dx_h * dx_h)), c->halo_grid, out, c->stream);
+                           (float)(1.0 / (dx_h * dx_h * dx_h)), c->halo_acc, out, c->stream);
   });
   if (mean && (rc = box_mean(c, out, c->n3, mean))) return rc;
   if (hipStreamSynchronize(c->stream) != hipSuccess) return SF21_ERR_HIP;
@@ -2095,6 +2072,7 @@ int sf21_nldensity_dev(sf21_hii_ctx* c, const sf21_params* p, double z, const fl
   // get_nldensity.c:95-99, :117, :132: velocities to cells (box_len in
   // Mpc/h, the files in Mpc), the z = 0 mass 1 + delta0 D(300), the
   // displacement factor D(z) - D(300)
+  if (!deposit_prepare()) return SF21_ERR_HIP;
   const double growth_in = sf21_growth(p, 300.0);
   const double growth = sf21_growth(p, z) - growth_in;
   const double vscale = (double)ng / p->box_len * p->hubble;
