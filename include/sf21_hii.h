@@ -78,7 +78,8 @@ typedef struct sf21_hii_config {
   int radius_batch;      /* radii per fused filter pass, 0 = automatic (the whole ladder
                             while its K n^3 complex buffer takes at most a third of the
                             free device memory, else fewer, 16 at least if they fit);
-                            sides without a register plan run one radius per step */
+                            sides without a register plan batch by themselves (at most
+                            16 GiB and a third of the free memory) and report 1 */
   int device;            /* HIP device ordinal */
   int filter_tile;       /* columns per block of the fused filter pass: 4, 8, 16 or 0 (auto) */
   int filter_w;          /* top-hat weights W(|k| R): 0 = automatic (FP32),
@@ -280,7 +281,7 @@ int sf21_hii_filtered_dev(sf21_hii_ctx *ctx, const float *a, const float *b, con
  * (device arch, n, box_len, the radii).  A context created with
  * radius_batch, filter_tile and filter_w all 0 takes the cached choice for
  * its key from $SF21_TUNE_CACHE.  *best_ms (nullable): the winner's time per
- * slice.  Sides without a register plan (one radius per step through line
+ * slice.  Sides without a register plan (line
  * transforms) have one choice: which column passes (along j, along i) deal
  * runs of consecutive blocks to one XCD (sf21_hii_line_order); the four
  * masks are timed and the winner is cached the same way.  Every choice

@@ -39,19 +39,28 @@ struct GenPlan {
 // Whole-line transforms (first and last stage in HBM, the others through
 // LDS), 8 lines per 256-thread block: axis 0
 // along p (contiguous rows), 1 along j, 2 along i (8 adjacent p columns).
-// mode 0: in place (src == dst allowed); 1 (axis 2 only): inverse-filter
-// input -- each element of src times W(|k| R) (kappa = dk R as hi + lo)
-// before the transform, result to dst; 2: centre test after the transform (Re = n^3
-// rec_R, Im = s n^3 ion_R, s = bal[0]): wmap = d2 where a centre, nothing
-// stored (dst null); 3: dst = (Re, Im / s), the unscaled filtered pair (the
-// same kernel as mode 2).  LDS: gen_pass_lds(plan) bytes.
+// mode 0: in place (src == dst allowed); 1 (axis 2, inverse): each element of
+// src times W(|k| R) (kappa = dk R as hi + lo) before the transform, result to
+// dst.  LDS: gen_pass_lds(plan) bytes.
 bool gen_plan_make(int n, GenPlan* p);
 size_t gen_pass_lds(const GenPlan& p);
 // allows the transform blocks' LDS on the current device (false: refused)
 bool gen_prepare(const GenPlan& p);
 void launch_gen_pass(const GenPlan& plan, int axis, int sign, int mode, const float2* src,
-                     float2* dst, const float2* tw, float2 kappa, const float* bal, int* wmap,
-                     int d2, hipStream_t s);
+                     float2* dst, const float2* tw, float2 kappa, hipStream_t s);
+// The finder's passes over nrad radii, specialised per side, per-radius
+// buffer u of n^3 pairs each in tiles (kernels_generic.hip): filtered inverse
+// along i from the full spectrum and the radii's weight table; inverse along
+// j in place (not on plane sides); inverse along p (plane sides: j and p) with
+// the centre test, dbg (nullable, one radius): the unscaled pairs instead of
+// the map.
+bool gen_finder_prepare(int n);
+bool gen_plane_side(int n);
+void launch_gen_filter(const GenPlan& plan, const float2* spec, float2* u, int nrad, const float* wt,
+                       const float2* tw, hipStream_t s);
+void launch_gen_inv_j(const GenPlan& plan, float2* u, int nrad, const float2* tw, hipStream_t s);
+void launch_gen_crit(const GenPlan& plan, const float2* u, int nrad, const int* d2max,
+                     const float* bal, int* wmap, float2* dbg, const float2* tw, hipStream_t s);
 // spec = (rec, s ion) of the cell pre-pass, s = bal[0]
 void launch_gen_pack(long n3, const float* a, const float* b, const float* c, CellConsts k,
                      const float* bal, float2* spec, hipStream_t s);
@@ -81,8 +90,9 @@ struct FilterW {
   const float* table;
   const float2* kappa;
 };
-// floats of one radius of the weight table: [fj][p/16][fi][p%16]
-constexpr long wtab_radius(int n) { return (long)(n / 2 + 1) * (n / 2 + 1) * ((n + 15) / 16 * 16); }
+// floats of one radius of the weight table: [fj][p/g][fi][p%g], g = 16, or 8
+// on sides that are an odd multiple of 8
+constexpr long wtab_radius(int n) { return (long)(n / 2 + 1) * (n / 2 + 1) * n; }
 void launch_w_table(int n, int nr, const float2* kappa, float* wt, hipStream_t s);
 // radii rb .. rb + nrad - 1 of the ladder; mirror: the block order that runs
 // the i-lines kj and n - kj, which share their weights, together on one XCD;

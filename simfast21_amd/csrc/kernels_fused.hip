@@ -268,18 +268,19 @@ __global__ __launch_bounds__(TILE*(L / E)) void k_cols_pipe(const float2* in, fl
 
 // ------------------------------------------------------------------------
 // Top-hat weights of every radius, laid out as the filter passes read them:
-// wt[r][fj][p/16][fi][p%16] (fj, fi <= n/2 the folded frequencies along j and
-// i): a block's weights of one radius are one contiguous piece of whole cache
-// lines.  The same function of the same integer |k|^2 as an evaluation in the
-// filter pass, so the same values; computed once per context.
+// wt[r][fj][p/g][fi][p%g] (fj, fi <= n/2 the folded frequencies along j and i;
+// g = 16, or 8 on sides that are an odd multiple of 8): a block's weights of
+// one radius are one contiguous piece of whole cache lines.  The same function
+// of the same integer |k|^2 as an evaluation in the filter pass, so the same
+// values; computed once per context.
 // ------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_w_table(int n, const float2* __restrict__ kappa,
                                                  float* __restrict__ wt) {
-  const int H = n / 2 + 1, ct = (n + 15) / 16;
+  const int H = n / 2 + 1, g = n % 16 == 0 ? 16 : 8;
   const int pt = blockIdx.x, fj = blockIdx.y, r = blockIdx.z;
-  float* __restrict__ blk = wt + (((long)r * H + fj) * ct + pt) * (H * 16);
-  for (int e = threadIdx.x; e < H * 16; e += blockDim.x) {
-    const int fi = e >> 4, p = pt * 16 + (e & 15);
+  float* __restrict__ blk = wt + (((long)r * H + fj) * (n / g) + pt) * (H * g);
+  for (int e = threadIdx.x; e < H * g; e += blockDim.x) {
+    const int fi = e / g, p = pt * g + e % g;
     blk[e] = w_tophat_k(kappa[r], fj * fj + fi * fi + fold_sq(p, n));
   }
 }
@@ -1049,7 +1050,8 @@ static int radius_groups(long waves, int nrad) {
 }
 
 void launch_w_table(int n, int nr, const float2* kappa, float* wt, hipStream_t s) {
-  hipLaunchKernelGGL(k_w_table, dim3((n + 15) / 16, n / 2 + 1, nr), dim3(256), 0, s, n, kappa, wt);
+  const int g = n % 16 == 0 ? 16 : 8;
+  hipLaunchKernelGGL(k_w_table, dim3(n / g, n / 2 + 1, nr), dim3(256), 0, s, n, kappa, wt);
 }
 
 void launch_filter_i(int n, const float2* spec, float2* u, int nrad, long ustride,

@@ -128,6 +128,8 @@ struct sf21_hii_ctx {
   float* wlut = nullptr;
   long mlut = 0;
   float* wtab = nullptr;  // FP32 top-hat weights per radius (wtab_radius floats each)
+  bool wtab_all = false;  // wtab holds every radius (else one batch, filled per batch)
+  int Kg = 1;             // generic sides: radii per batch
   bool plane = false;     // j and p inverses and centre test plane by plane
   int* d_d2 = nullptr;
   // fused path
@@ -305,10 +307,10 @@ int check_hip() {
   return e == hipSuccess ? SF21_OK : SF21_ERR_HIP;
 }
 
-// ---- fused exact path on a generic side: one radius per step ------------
-// Forward transforms of z = rec + i s ion along p, j, i; per radius in
-// ascending order, the filtered inverse along i, the inverse along j and the
-// inverse along p with the centre test; then the same dilation and final
+// ---- fused exact path on a generic side ---------------------------------
+// Forward transforms of z = rec + i s ion along p, j, i; per batch of Kg radii
+// in ascending order, the filtered inverse along i, the inverse along j and
+// the inverse along p with the centre test; then the same dilation and final
 // pass as the register-plan sides.
 void enqueue_generic(sf21_hii_ctx* c, const float* a, const float* b, const float* cc, double z,
                      float* xhii, double* neutral_slot, int only_radius, float2* dbg) {
@@ -320,24 +322,21 @@ void enqueue_generic(sf21_hii_ctx* c, const float* a, const float* b, const floa
   launch(c, "balance", [&] { launch_balance(n3, a, b, cc, k, c->bal_part, c->bal, s); });
   launch(c, "gen_pack", [&] { launch_gen_pack(n3, a, b, cc, k, c->bal, c->spec, s); });
   for (int axis = 0; axis < 3; ++axis)
-    launch(c, "gen_fwd", [&] {
-      launch_gen_pass(g, axis, -1, 0, c->spec, c->spec, c->tw, none, nullptr, nullptr, 0, s);
-    });
+    launch(c, "gen_fwd", [&] { launch_gen_pass(g, axis, -1, 0, c->spec, c->spec, c->tw, none, s); });
   launch(c, "fill_map", [&] { launch_fill_i32(c->wmap, -1, n3, s); });
   const int r_lo = only_radius >= 0 ? only_radius : 0;
   const int r_hi = only_radius >= 0 ? only_radius + 1 : (int)c->radii.size();
-  for (int r = r_hi - 1; r >= r_lo; --r) {
-    launch(c, "gen_filter_i", [&] {
-      launch_gen_pass(g, 2, +1, 1, c->spec, c->ubuf, c->tw, c->kap[r], nullptr, nullptr, 0, s);
-    });
-    launch(c, "gen_inv_j", [&] {
-      launch_gen_pass(g, 1, +1, 0, c->ubuf, c->ubuf, c->tw, none, nullptr, nullptr, 0, s);
-    });
+  for (int re = r_hi; re > r_lo; re -= c->Kg) {
+    const int rb = std::max(r_lo, re - c->Kg);
+    const int kk = re - rb;
+    const float* wt = c->wtab + (c->wtab_all ? rb * wtab_radius(c->n) : 0);
+    if (!c->wtab_all)
+      launch(c, "w_table", [&] { launch_w_table(c->n, kk, c->d_kappa + rb, c->wtab, s); });
+    launch(c, "gen_filter_i", [&] { launch_gen_filter(g, c->spec, c->ubuf, kk, wt, c->tw, s); });
+    if (!gen_plane_side(c->n))
+      launch(c, "gen_inv_j", [&] { launch_gen_inv_j(g, c->ubuf, kk, c->tw, s); });
     launch(c, "gen_inv_p_crit", [&] {
-      if (dbg)
-        launch_gen_pass(g, 0, +1, 3, c->ubuf, dbg, c->tw, none, c->bal, nullptr, 0, s);
-      else
-        launch_gen_pass(g, 0, +1, 2, c->ubuf, nullptr, c->tw, none, c->bal, c->wmap, c->d2[r], s);
+      launch_gen_crit(g, c->ubuf, kk, c->d_d2 + rb, c->bal, c->wmap, dbg, c->tw, s);
     });
   }
   if (only_radius >= 0) return;
@@ -569,7 +568,7 @@ void enqueue_pk(sf21_hii_ctx* c, const float* field, float2* half, int nbins) {
     launch(c, "to_complex", [&] { launch_to_complex(c->n3, field, half, s); });
     for (int axis = 0; axis < 3; ++axis)
       launch(c, "gen_fwd", [&] {
-        launch_gen_pass(c->gplan, axis, -1, 0, half, half, c->tw, none, nullptr, nullptr, 0, s);
+        launch_gen_pass(c->gplan, axis, -1, 0, half, half, c->tw, none, s);
       });
   } else {
     r2c3d(c, field, half);
@@ -589,7 +588,7 @@ void gen_fft3(sf21_hii_ctx* c, float2* x, int sign) {
   const float2 none = make_float2(0.f, 0.f);
   for (int axis = 0; axis < 3; ++axis)
     launch(c, sign < 0 ? "gen_fwd" : "gen_inv", [&] {
-      launch_gen_pass(c->gplan, axis, sign, 0, x, x, c->tw, none, nullptr, nullptr, 0, c->stream);
+      launch_gen_pass(c->gplan, axis, sign, 0, x, x, c->tw, none, c->stream);
     });
 }
 
@@ -795,10 +794,10 @@ void enqueue_diff_backward_generic(sf21_hii_ctx* c, const float* g, const float*
   // the real-space pair (N R_R, s N I_R) of radius r into ubuf
   auto pair_of = [&](int r) {
     launch(c, "gen_filter_i", [&] {
-      launch_gen_pass(gp, 2, +1, 1, c->spec, c->ubuf, c->tw, c->kap[r], nullptr, nullptr, 0, s);
+      launch_gen_pass(gp, 2, +1, 1, c->spec, c->ubuf, c->tw, c->kap[r], s);
     });
-    launch(c, "gen_inv_j", [&] { launch_gen_pass(gp, 1, +1, 0, c->ubuf, c->ubuf, c->tw, none, nullptr, nullptr, 0, s); });
-    launch(c, "gen_inv_p", [&] { launch_gen_pass(gp, 0, +1, 0, c->ubuf, c->ubuf, c->tw, none, nullptr, nullptr, 0, s); });
+    launch(c, "gen_inv_j", [&] { launch_gen_pass(gp, 1, +1, 0, c->ubuf, c->ubuf, c->tw, none, s); });
+    launch(c, "gen_inv_p", [&] { launch_gen_pass(gp, 0, +1, 0, c->ubuf, c->ubuf, c->tw, none, s); });
   };
   // sweep 1: C = sum_R B_R FFT(phi_R)
   launch(c, "diff_fill", [&] { launch_fill_c(c->df_c, n3, s); });
@@ -1183,7 +1182,8 @@ int sf21_hii_create(const sf21_hii_config* cfg, sf21_hii_ctx** out) {
   c->dx = c->L / c->n;
   c->dk = 2 * kPi / c->L;
   c->generic = cfg->path == SF21_PATH_FUSED && !plan_size(c->n) && c->n != 32;
-  if (c->generic && (!gen_plan_make(c->n, &c->gplan) || !gen_prepare(c->gplan))) {
+  if (c->generic && (!gen_plan_make(c->n, &c->gplan) || !gen_prepare(c->gplan) ||
+                     !gen_finder_prepare(c->n))) {
     (void)hipGetLastError();
     delete c;
     return SF21_ERR_HIP;
@@ -1282,16 +1282,26 @@ int sf21_hii_create(const sf21_hii_config* cfg, sf21_hii_ctx** out) {
       rc = SF21_ERR_HIP;
       goto fail;
     }
-    if (c->filter_w && !c->generic) {
-      // the FP32 weight table, if it takes at most 1/16 of
-      // the free memory (otherwise the filter pass evaluates the weights)
-      const size_t count = (size_t)wtab_radius(c->n) * c->radii.size();
+    if (c->filter_w) {
+      // the FP32 weight table, if it takes at most 1/16 of the free memory
+      // (otherwise the filter pass evaluates the weights; generic sides fill a
+      // table of one batch, at most 16 GiB of pairs, before each batch)
+      const size_t nr = c->radii.size(), one = (size_t)wtab_radius(c->n);
       size_t free_b = 0, total_b = 0;
-      if (hipMemGetInfo(&free_b, &total_b) == hipSuccess && sizeof(float) * count <= free_b / 16 &&
-          dev_alloc(&c->wtab, count) == SF21_OK)
-        launch_w_table(c->n, (int)c->radii.size(), c->d_kappa, c->wtab, c->stream);
-      else
-        (void)hipGetLastError();
+      if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = 0;
+      if (sizeof(float) * one * nr <= free_b / 16 && dev_alloc(&c->wtab, one * nr) == SF21_OK) {
+        c->wtab_all = true;
+        launch_w_table(c->n, (int)nr, c->d_kappa, c->wtab, c->stream);
+      }
+      if (c->generic) {
+        c->Kg = (int)nr;
+        const size_t pair = sizeof(float2) * (size_t)c->n3;
+        while (c->Kg > 1 && (pair * c->Kg > ((size_t)16 << 30) || pair * c->Kg > free_b / 3))
+          c->Kg = (c->Kg + 1) / 2;
+        if (!c->wtab_all)
+          while ((rc = dev_alloc(&c->wtab, one * c->Kg)) && c->Kg > 1) c->Kg = (c->Kg + 1) / 2;
+        if (rc) goto fail;
+      }
     }
     if ((rc = dev_alloc(&c->d_d2, c->d2.size()))) goto fail;
     if (hipMemcpy(c->d_d2, c->d2.data(), sizeof(int) * c->d2.size(), hipMemcpyHostToDevice) !=
@@ -1321,8 +1331,11 @@ int sf21_hii_create(const sf21_hii_config* cfg, sf21_hii_ctx** out) {
     if (cfg->path == SF21_PATH_PLAIN) c->K = 1;
     if ((rc = dev_alloc(&c->spec, (size_t)c->n3))) goto fail;
     // automatic batch: halve K until the K n^3 complex buffer fits
-    while ((rc = dev_alloc(&c->ubuf, (size_t)c->n3 * c->K)) && cfg->radius_batch <= 0 && c->K > 1)
-      c->K /= 2;
+    if (c->generic)
+      while ((rc = dev_alloc(&c->ubuf, (size_t)c->n3 * c->Kg)) && c->Kg > 1) c->Kg = (c->Kg + 1) / 2;
+    else
+      while ((rc = dev_alloc(&c->ubuf, (size_t)c->n3 * c->K)) && cfg->radius_batch <= 0 && c->K > 1)
+        c->K /= 2;
     if (rc) goto fail;
     if (c->Kd > c->K) c->Kd = c->K;
     if ((rc = dev_alloc(&c->wmap, (size_t)c->n3)) || (rc = dev_alloc(&c->gbuf, (size_t)c->n3)) ||
@@ -1966,12 +1979,12 @@ int sf21_t21_dev(sf21_hii_ctx* c, const sf21_params* p, double z, const float* d
     launch(c, "to_complex", [&] { launch_to_complex(n3, delta, c->spec, s); });
     for (int axis = 0; axis < 3; ++axis)
       launch(c, "gen_fwd", [&] {
-        launch_gen_pass(c->gplan, axis, -1, 0, c->spec, c->spec, c->tw, none, nullptr, nullptr, 0, s);
+        launch_gen_pass(c->gplan, axis, -1, 0, c->spec, c->spec, c->tw, none, s);
       });
     launch(c, "vgrad_filter", [&] { launch_vgrad_filter_full(n, c->spec, p->vel_comp, s); });
     for (int axis = 0; axis < 3; ++axis)
       launch(c, "gen_inv", [&] {
-        launch_gen_pass(c->gplan, axis, +1, 0, c->spec, c->spec, c->tw, none, nullptr, nullptr, 0, s);
+        launch_gen_pass(c->gplan, axis, +1, 0, c->spec, c->spec, c->tw, none, s);
       });
     launch(c, "real_part", [&] { launch_real_part(n3, c->spec, c->t21_dv, s); });
   } else {
