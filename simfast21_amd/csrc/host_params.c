@@ -6,7 +6,7 @@
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
-#include "../../include/sf21_hii.h"
+#include "host_params.h"
 
 #define SF21_PI 3.1415926535897932385E0 /* Input_variables.h:10 */
 
@@ -119,24 +119,126 @@ double sf21_hubble_z(const sf21_params *p, double z) {
   return p->hubble * SF21_H0 * sqrt(p->omega_m * (1. + z) * (1. + z) * (1. + z) + p->omega_lambda);
 }
 
-static double growth_integral(const sf21_params *p, double zz) {
-  const double dz = 0.001, h0 = sf21_hubble_z(p, 0.);
-  double s = 0., z, e;
-  for (z = zz + dz / 2.; z < zz + 100.; z += dz) {
-    e = sf21_hubble_z(p, z) / h0;
-    s += (1. + z) / e / e / e;
+/* Midpoints z, z + dz, ... below end, each the rounded sum of the one before
+ * and dz.  Inside a binade the spacing of the doubles is constant, so every
+ * addition of dz advances by the same multiple d of it (once two steps in a row
+ * agree: a tie, dz half way between two multiples, goes by the parity, which
+ * then no longer changes) and z + m d is exact: runs of values without the
+ * chain of additions. */
+#define GROWTH_DZ 0.001
+#define GROWTH_BLOCK 256
+typedef struct {
+  double z, end, d;
+  long left; /* values left in the run */
+} growth_seq;
+
+static int growth_fill(growth_seq *q, double *zs) {
+  int n = 0;
+  while (n < GROWTH_BLOCK && q->z < q->end) {
+    if (q->left == 0) {
+      const double z = q->z, d = (z + GROWTH_DZ) - z, z1 = z + d;
+      if (z1 == z) { /* dz below the spacing at z */
+        q->z = q->end;
+        break;
+      }
+      q->left = 1;
+      if (z >= 0x1p-6 && (z1 + GROWTH_DZ) - z1 == d) {
+        const double top = ldexp(1.0, ilogb(z) + 1), lim = top < q->end ? top : q->end;
+        long c = (long)((lim - z) / d);
+        while (c > 1 && !(z + (c - 1) * d < lim)) c--;
+        while (z + c * d < lim) c++;
+        if (c > 1) q->left = c;
+      }
+      q->d = d;
+    }
+    const int c = q->left < GROWTH_BLOCK - n ? (int)q->left : GROWTH_BLOCK - n;
+    for (int m = 0; m < c; m++) zs[n + m] = q->z + m * q->d;
+    n += c;
+    q->left -= c;
+    q->z = q->left ? q->z + c * q->d : zs[n - 1] + GROWTH_DZ;
   }
-  return s * dz;
+  return n;
+}
+
+/* (1+z)/(H(z)/H(0))^3 of a block, zero behind its n values: one square root
+ * and four divisions a term, in vector units where the CPU has wide ones.
+ * Every operation rounds by itself, as in a loop over single values. */
+static inline __attribute__((always_inline)) void growth_terms_body(const sf21_params *p, double h0,
+                                                                    int n, double *zt) {
+  const double om = p->omega_m, ol = p->omega_lambda, a = p->hubble * SF21_H0;
+  for (int m = n; m < GROWTH_BLOCK; m++) zt[m] = 0.;
+  for (int m = 0; m < GROWTH_BLOCK; m++) {
+    const double z = zt[m], z1 = 1. + z;
+    const double e = a * sqrt(om * z1 * z1 * z1 + ol) / h0;
+    zt[m] = z1 / e / e / e;
+  }
+  for (int m = n; m < GROWTH_BLOCK; m++) zt[m] = 0.;
+}
+static void growth_terms_base(const sf21_params *p, double h0, int n, double *zt) {
+  growth_terms_body(p, h0, n, zt);
+}
+#ifdef __x86_64__
+__attribute__((target("avx2"))) static void growth_terms_avx2(const sf21_params *p, double h0, int n,
+                                                              double *zt) {
+  growth_terms_body(p, h0, n, zt);
+}
+__attribute__((target("avx512f,prefer-vector-width=512"))) static void growth_terms_avx512(
+    const sf21_params *p, double h0, int n, double *zt) {
+  growth_terms_body(p, h0, n, zt);
+}
+#endif
+
+/* D(z[k]), k < nz <= 3, in one sweep together with the integral at 0: the
+ * sums, chains of dependent additions in ascending z, run side by side.  Bound
+ * by the divider: an integral of 1e5 terms 0.085 ms with 512-bit vectors, 0.145
+ * with 256-bit ones, 0.48 one value at a time (EPYC). */
+void sf21_growth_many(const sf21_params *p, int nz, const double *z, double *growth) {
+  void (*terms)(const sf21_params *, double, int, double *) = growth_terms_base;
+  const double h0 = sf21_hubble_z(p, 0.);
+  double s[4] = {0., 0., 0., 0.};
+  double buf[4][GROWTH_BLOCK];
+  growth_seq q[4];
+  int more = 1;
+#ifdef __x86_64__
+  if (__builtin_cpu_supports("avx512f")) terms = growth_terms_avx512;
+  else if (__builtin_cpu_supports("avx2")) terms = growth_terms_avx2;
+#endif
+  memset(buf, 0, sizeof(buf));
+  for (int k = 0; k <= nz; k++) {
+    const double zz = k < nz ? z[k] : 0.;
+    q[k] = (growth_seq){zz + GROWTH_DZ / 2., zz + 100., 0., 0};
+  }
+  while (more) {
+    more = 0;
+    for (int k = 0; k <= nz; k++) {
+      const int n = growth_fill(&q[k], buf[k]);
+      terms(p, h0, n, buf[k]);
+      if (n) more = 1;
+    }
+    if (more)
+      for (int m = 0; m < GROWTH_BLOCK; m++)
+        for (int k = 0; k < 4; k++) s[k] += buf[k][m];
+  }
+  for (int k = 0; k < nz; k++)
+    growth[k] = sf21_hubble_z(p, z[k]) / h0 * (s[k] * GROWTH_DZ) / (s[nz] * GROWTH_DZ);
 }
 
 double sf21_growth(const sf21_params *p, double z) {
-  return sf21_hubble_z(p, z) / sf21_hubble_z(p, 0.) * growth_integral(p, z) / growth_integral(p, 0.);
+  double d;
+  sf21_growth_many(p, 1, &z, &d);
+  return d;
+}
+
+/* from D(z + dz/2) and D(z - dz/2) */
+double sf21_dgrowth_of(const sf21_params *p, double z, double hi, double lo) {
+  return (hi - lo) / GROWTH_DZ * (-sf21_hubble_z(p, z) * (1. + z));
 }
 
 double sf21_dgrowth_dt(const sf21_params *p, double z) {
-  const double dz = 1e-3;
-  return (sf21_growth(p, z + dz / 2.) - sf21_growth(p, z - dz / 2.)) / dz *
-         (-sf21_hubble_z(p, z) * (1. + z));
+  const double zs[2] = {z + GROWTH_DZ / 2., z - GROWTH_DZ / 2.};
+  double d[2];
+  sf21_growth_many(p, 2, zs, d);
+  return sf21_dgrowth_of(p, z, d[0], d[1]);
 }
 
 int sf21_ladder(double rmax, double dx, int nbins, double *radii, int cap, int *n_main) {

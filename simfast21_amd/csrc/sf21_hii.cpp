@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "../../include/sf21_hii.h"
+#include "host_params.h"
 #include "kernels.h"
 
 using namespace sf21;
@@ -1964,14 +1965,6 @@ int sf21_t21_dev(sf21_hii_ctx* c, const sf21_params* p, double z, const float* d
   if (!c->t21_dv && ((rc = dev_alloc(&c->t21_dv, (size_t)n3)) ||
                      (rc = dev_alloc(&c->t21_part, (size_t)2 * t21_partials_count(n3) + 2))))
     return rc;
-  // per-redshift scalars in FP64 (auxiliary.c:224-292, t21.c:197-212)
-  const double growth = sf21_growth(p, z), dgdt = sf21_dgrowth_dt(p, z), hz = sf21_hubble_z(p, z);
-  const double h = p->hubble;
-  const double c21 = 23.0 / 1000. * (0.7 / h) * (p->omega_b * h * h / 0.02) *
-                     std::sqrt((0.15 / p->omega_m / h / h) * (1. + z) / 10.);
-  // -dD/dt / (H D) times the unnormalised transform's 1/N^3 (dx^3/L^3)
-  const double vfac = -dgdt / hz / growth / (double)n3;
-  const double tcmb = 2.725 * (1. + z);
   if (c->generic) {
     // complex transforms of the real box through the generic line passes
     hipStream_t s = c->stream;
@@ -1992,6 +1985,18 @@ int sf21_t21_dev(sf21_hii_ctx* c, const sf21_params* p, double z, const float* d
     launch(c, "vgrad_filter", [&] { launch_vgrad_filter(n, c->spec, p->vel_comp, c->stream); });
     c2r3d(c, c->spec, c->t21_dv);
   }
+  // per-redshift scalars in FP64 (auxiliary.c:224-292, t21.c:197-212)
+  // while the transforms run
+  const double dzh = 0.5e-3, zs[3] = {z, z + dzh, z - dzh};
+  double gs[3];
+  sf21_growth_many(p, 3, zs, gs);
+  const double growth = gs[0], dgdt = sf21_dgrowth_of(p, z, gs[1], gs[2]), hz = sf21_hubble_z(p, z);
+  const double h = p->hubble;
+  const double c21 = 23.0 / 1000. * (0.7 / h) * (p->omega_b * h * h / 0.02) *
+                     std::sqrt((0.15 / p->omega_m / h / h) * (1. + z) / 10.);
+  // -dD/dt / (H D) times the unnormalised transform's 1/N^3 (dx^3/L^3)
+  const double vfac = -dgdt / hz / growth / (double)n3;
+  const double tcmb = 2.725 * (1. + z);
   double* sums = c->t21_part + 2 * t21_partials_count(n3);
   launch(c, "t21_cells", [&] {
     launch_t21_cells(n3, delta, xhii, c->t21_dv, xc, xalpha, tk, (float)vfac, (float)c21,
@@ -2086,8 +2091,10 @@ int sf21_nldensity_dev(sf21_hii_ctx* c, const sf21_params* p, double z, const fl
   // Mpc/h, the files in Mpc), the z = 0 mass 1 + delta0 D(300), the
   // displacement factor D(z) - D(300)
   if (!deposit_prepare()) return SF21_ERR_HIP;
-  const double growth_in = sf21_growth(p, 300.0);
-  const double growth = sf21_growth(p, z) - growth_in;
+  const double zs[2] = {300.0, z};
+  double gs[2];
+  sf21_growth_many(p, 2, zs, gs);
+  const double growth_in = gs[0], growth = gs[1] - growth_in;
   const double vscale = (double)ng / p->box_len * p->hubble;
   launch(c, "nldensity", [&] {
     launch_nldensity(ng, ns, (int)sm, vx, vy, vz, delta0, (float)vscale, (float)growth_in,
