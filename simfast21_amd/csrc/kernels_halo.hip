@@ -120,112 +120,144 @@ __global__ void k_fill_value(float* __restrict__ p, float value, long count) {
 // A block takes a tile of source cells.  Neighbouring cells move together, so
 // the tile lands in a box little larger than itself: where that box fits the
 // block's LDS the deposits are added there and every touched cell then takes
-// one global atomic, in rows of consecutive addresses -- about 2 per source
-// cell instead of 8.  A tile whose cells scatter farther (or hold a NaN)
-// deposits directly.  512^3, displacements of 1.1 cells rms: 24.7 ms direct,
-// 6.1 ms this way.  Bound: the global atomics (43e9 a second either way).
-constexpr int kDepTX = 16, kDepTY = 16, kDepTZ = 32, kDepThreads = 512;
-constexpr int kDepCap = 19456;  // floats: two blocks per CU
+// one global atomic, in rows of consecutive addresses -- about 3 per source
+// cell instead of 8.  The LDS sums are FP64: an FP32 LDS atomic takes 193
+// cycles a wave here, an FP64 one 9.  A tile whose cells scatter farther (or
+// hold a NaN) deposits directly.  Blocks stay and take one tile after another,
+// the next one's velocities loaded while this one is added up.  512^3,
+// displacements of 1.1 cells rms: 24.7 ms direct, 6.1 with FP32 sums in tiles of
+// 16 x 16 x 32, 2.1 this way (2.5 with a block per tile).  Tried and slower: tiles by
+// parity in 8 launches with plain additions to the grid, 2.8 ms.  Bound: the
+// global atomics, 2e11 a second, and the phases of one block per CU.
+constexpr int kDepTX = 16, kDepTY = 16, kDepTZ = 16, kDepThreads = 1024;
+constexpr int kDepCells = kDepTX * kDepTY * kDepTZ / kDepThreads;  // of a thread, in registers
+constexpr int kDepCap = 19968;  // doubles: one block per CU
+constexpr long kDepBlocks = 256;  // one per CU
 
 __global__ __launch_bounds__(kDepThreads) void k_displace_deposit(
-    int ng, const float* __restrict__ vx, const float* __restrict__ vy, const float* __restrict__ vz,
-    const float* __restrict__ delta0, float vscale, float growth_in, float growth,
-    float* __restrict__ grid) {
-  extern __shared__ float box[];
+    int ng, int tiles, const float* __restrict__ vx, const float* __restrict__ vy,
+    const float* __restrict__ vz, const float* __restrict__ delta0, float vscale, float growth_in,
+    float growth, float* __restrict__ grid) {
+  extern __shared__ double box[];
   __shared__ int lo[3], hi[3];
   const int nty = (ng + kDepTY - 1) / kDepTY, ntz = (ng + kDepTZ - 1) / kDepTZ;
-  const int i0 = blockIdx.x / (nty * ntz) * kDepTX, j0 = blockIdx.x / ntz % nty * kDepTY,
-            p0 = blockIdx.x % ntz * kDepTZ;
   const int tid = threadIdx.x;
-  if (tid < 3) {
-    lo[tid] = INT_MAX;
-    hi[tid] = INT_MIN;
-  }
-  __syncthreads();
-  // the tile's cells, p fastest; f(index, displaced position)
-  auto each = [&](auto&& f) {
-    for (int e = tid; e < kDepTX * kDepTY * kDepTZ; e += kDepThreads) {
-      const int i = i0 + e / (kDepTY * kDepTZ), j = j0 + e / kDepTZ % kDepTY, p = p0 + e % kDepTZ;
-      if (i >= ng || j >= ng || p >= ng) continue;
+  // the thread's cells of a tile, p fastest over the threads
+  auto cell = [&](int tile, int u, int& i, int& j, int& p) {
+    const int e = tid + u * kDepThreads;
+    i = tile / (nty * ntz) * kDepTX + e / (kDepTY * kDepTZ);
+    j = tile / ntz % nty * kDepTY + e / kDepTZ % kDepTY;
+    p = tile % ntz * kDepTZ + e % kDepTZ;
+    return i < ng && j < ng && p < ng;
+  };
+  float v[kDepCells][4] = {};
+  auto load = [&](int tile) {
+#pragma unroll
+    for (int u = 0; u < kDepCells; ++u) {
+      int i, j, p;
+      if (!cell(tile, u, i, j, p)) continue;
       const long ind = ((long)i * ng + j) * ng + p;
-      f(ind, fmaf(vx[ind] * vscale, growth, (float)i), fmaf(vy[ind] * vscale, growth, (float)j),
-        fmaf(vz[ind] * vscale, growth, (float)p));
+      v[u][0] = vx[ind];
+      v[u][1] = vy[ind];
+      v[u][2] = vz[ind];
+      v[u][3] = delta0[ind];
     }
   };
-  int mn[3] = {INT_MAX, INT_MAX, INT_MAX}, mx[3] = {INT_MIN, INT_MIN, INT_MIN};
-  each([&](long, float x1, float y1, float z1) {
-    const float r[3] = {x1, y1, z1};
+  if ((int)blockIdx.x < tiles) load(blockIdx.x);
+  for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+    if (tid < 3) {
+      lo[tid] = INT_MAX;
+      hi[tid] = INT_MIN;
+    }
+    __syncthreads();
+    float r[kDepCells][3], m[kDepCells];  // displaced positions, masses
+    bool in[kDepCells];
+    int mn[3] = {INT_MAX, INT_MAX, INT_MAX}, mx[3] = {INT_MIN, INT_MIN, INT_MIN};
+#pragma unroll
+    for (int u = 0; u < kDepCells; ++u) {
+      int c[3];
+      in[u] = cell(tile, u, c[0], c[1], c[2]);
+      m[u] = fmaf(v[u][3], growth_in, 1.0f);
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        r[u][a] = fmaf(v[u][a] * vscale, growth, (float)c[a]);
+        int q;
+        float far;
+        cic_axis(r[u][a], q, far);
+        if (in[u]) {
+          mn[a] = min(mn[a], q);
+          mx[a] = max(mx[a], q);
+        }
+      }
+    }
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-      int c;
-      float far;
-      cic_axis(r[a], c, far);
-      mn[a] = min(mn[a], c);
-      mx[a] = max(mx[a], c);
-    }
-  });
 #pragma unroll
-  for (int a = 0; a < 3; ++a) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      mn[a] = min(mn[a], __shfl_xor(mn[a], o, 64));
-      mx[a] = max(mx[a], __shfl_xor(mx[a], o, 64));
-    }
-    if ((tid & 63) == 0) {
-      atomicMin(&lo[a], mn[a]);
-      atomicMax(&hi[a], mx[a]);
-    }
-  }
-  __syncthreads();
-  const int x0 = lo[0], y0 = lo[1], z0 = lo[2];
-  // cells lo .. hi + 1 along each axis; 64-bit: positions may be anything
-  const long ex = (long)hi[0] - x0 + 2, ey = (long)hi[1] - y0 + 2, ez = (long)hi[2] - z0 + 2;
-  // a full edge first: the product of the three stays below 2^62
-  const bool fits = ex <= kDepCap && ey <= kDepCap && ez <= kDepCap && ex * ey * ez <= kDepCap;
-  if (!fits) {
-    each([&](long ind, float x1, float y1, float z1) {
-      cic_deposit(x1, y1, z1, fmaf(delta0[ind], growth_in, 1.0f), ng, grid);
-    });
-    return;
-  }
-  const int dy = (int)ey, dz = (int)ez, vol = (int)(ex * ey * ez);
-  for (int e = tid; e < vol; e += kDepThreads) box[e] = 0.0f;
-  __syncthreads();
-  each([&](long ind, float x1, float y1, float z1) {
-    const float v = fmaf(delta0[ind], growth_in, 1.0f);
-    int x, y, z;
-    float fx, fy, fz;
-    cic_axis(x1, x, fx);
-    cic_axis(y1, y, fy);
-    cic_axis(z1, z, fz);
-    float* b = box + ((x - x0) * dy + (y - y0)) * dz + (z - z0);
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        const float w = (a ? fx : 1.0f - fx) * (c ? fy : 1.0f - fy);
-        float* r = b + (a * dy + c) * dz;
-        atomicAdd(r, w * (1.0f - fz) * v);
-        atomicAdd(r + 1, w * fz * v);
+      for (int o = 32; o > 0; o >>= 1) {
+        mn[a] = min(mn[a], __shfl_xor(mn[a], o, 64));
+        mx[a] = max(mx[a], __shfl_xor(mx[a], o, 64));
       }
-  });
-  __syncthreads();
-  // one wave per row of the box; offsets past a wrapped start: one
-  // subtraction unless the box is wider than the grid
-  const int xw = wrap_cell(x0, ng), yw = wrap_cell(y0, ng), zw = wrap_cell(z0, ng);
-  auto past = [ng](int w, int k) {
-    w += k;
-    if (w >= ng) w -= ng;
-    return w < ng ? w : w % ng;
-  };
-  const int rows = (int)(ex * ey);
-  for (int q = tid >> 6; q < rows; q += kDepThreads / 64) {
-    const long base = ((long)past(xw, q / dy) * ng + past(yw, q % dy)) * ng;
-    for (int k = tid & 63; k < dz; k += 64) {
-      const float v = box[q * dz + k];
-      // 0: nothing landed there, or nothing to add
-      if (v != 0.0f) atomicAdd(&grid[base + past(zw, k)], v);
+      if ((tid & 63) == 0) {
+        atomicMin(&lo[a], mn[a]);
+        atomicMax(&hi[a], mx[a]);
+      }
     }
+    if (tile + (int)gridDim.x < tiles) load(tile + gridDim.x);  // before this tile's atomics
+    __syncthreads();
+    const int x0 = lo[0], y0 = lo[1], z0 = lo[2];
+    // cells lo .. hi + 1 along each axis; 64-bit: positions may be anything
+    const long ex = (long)hi[0] - x0 + 2, ey = (long)hi[1] - y0 + 2, ez = (long)hi[2] - z0 + 2;
+    // a full edge first: the product of the three stays below 2^62
+    const bool fits = ex <= kDepCap && ey <= kDepCap && ez <= kDepCap && ex * ey * ez <= kDepCap;
+    if (!fits) {
+#pragma unroll
+      for (int u = 0; u < kDepCells; ++u)
+        if (in[u]) cic_deposit(r[u][0], r[u][1], r[u][2], m[u], ng, grid);
+      __syncthreads();  // lo and hi are read before the next tile resets them
+      continue;
+    }
+    const int dy = (int)ey, dz = (int)ez, vol = (int)(ex * ey * ez);
+    for (int e = tid; e < vol; e += kDepThreads) box[e] = 0.0;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kDepCells; ++u) {
+      if (!in[u]) continue;
+      int x, y, z;
+      float fx, fy, fz;
+      cic_axis(r[u][0], x, fx);
+      cic_axis(r[u][1], y, fy);
+      cic_axis(r[u][2], z, fz);
+      double* b = box + ((x - x0) * dy + (y - y0)) * dz + (z - z0);
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          const float w = (a ? fx : 1.0f - fx) * (c ? fy : 1.0f - fy);
+          double* q = b + (a * dy + c) * dz;
+          atomicAdd(q, (double)(w * (1.0f - fz) * m[u]));
+          atomicAdd(q + 1, (double)(w * fz * m[u]));
+        }
+    }
+    __syncthreads();
+    // offsets past a wrapped start: one subtraction unless the box is wider
+    // than the grid
+    const int xw = wrap_cell(x0, ng), yw = wrap_cell(y0, ng), zw = wrap_cell(z0, ng);
+    auto past = [ng](int w, int k) {
+      w += k;
+      if (w >= ng) w -= ng;
+      return w < ng ? w : w % ng;
+    };
+    // floor(e / n) for e < 2^15: (e + 1/2) / n lies 1/(2 n) or more inside an
+    // integer interval, the product's error is below 2^-7 / n
+    const float rdz = 1.0f / (float)dz, rdy = 1.0f / (float)dy;
+    for (int e = tid; e < vol; e += kDepThreads) {
+      const float s = (float)box[e];
+      const int q = (int)(((float)e + 0.5f) * rdz), a = (int)(((float)q + 0.5f) * rdy);
+      // 0: nothing landed there, or nothing to add
+      if (s != 0.0f)
+        atomicAdd(&grid[((long)past(xw, a) * ng + past(yw, q - a * dy)) * ng + past(zw, e - q * dz)], s);
+    }
+    __syncthreads();  // the box is read before the next tile clears it
   }
 }
 
@@ -315,7 +347,7 @@ bool deposit_prepare() {
   // LDS above 64 KiB is requested per kernel
   return hipFuncSetAttribute((const void*)k_displace_deposit,
                              hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (int)sizeof(float) * kDepCap) == hipSuccess;
+                             (int)sizeof(double) * kDepCap) == hipSuccess;
 }
 
 void launch_nldensity(int ng, int ns, int sm, const float* vx, const float* vy, const float* vz,
@@ -325,9 +357,9 @@ void launch_nldensity(int ng, int ns, int sm, const float* vx, const float* vy, 
   const long tiles = (long)((ng + kDepTX - 1) / kDepTX) * ((ng + kDepTY - 1) / kDepTY) *
                      ((ng + kDepTZ - 1) / kDepTZ);
   hipLaunchKernelGGL(k_fill_value, dim3(blocks_for(g3)), dim3(256), 0, s, grid, -1.0f, g3);
-  hipLaunchKernelGGL(k_displace_deposit, dim3((unsigned)tiles), dim3(kDepThreads),
-                     sizeof(float) * kDepCap, s, ng, vx, vy, vz, delta0, vscale, growth_in, growth,
-                     grid);
+  hipLaunchKernelGGL(k_displace_deposit, dim3((unsigned)(tiles < kDepBlocks ? tiles : kDepBlocks)),
+                     dim3(kDepThreads), sizeof(double) * kDepCap, s, ng, (int)tiles, vx, vy, vz,
+                     delta0, vscale, growth_in, growth, grid);
   if (out)
     hipLaunchKernelGGL(k_smooth_scale, dim3(blocks_for((long)ns * ns * ns)), dim3(256), 0, s, ng,
                        ns, sm, grid, 1.0f, out);
