@@ -68,7 +68,7 @@ void launch_gen_pack(long n3, const float* a, const float* b, const float* c, Ce
 // ---- fused exact path ----
 int balance_partials_count(long n3);
 void launch_balance(long n3, const float* a, const float* b, const float* c, CellConsts k,
-                    double* part, float* scale, hipStream_t s);
+                    double* part, float* scale, int* map, hipStream_t s);
 void launch_fwd_rows(int n, const float* a, const float* b, const float* c, CellConsts k,
                      const float* bal, float2* y, const float2* tw, hipStream_t s);
 // tile: columns per block (8, 16; 16 or 32 when wide); variant bit 0: 16

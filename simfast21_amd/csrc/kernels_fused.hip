@@ -30,12 +30,15 @@ namespace sf21 {
 // field inherits the larger one's absolute error.  s = 2^round(log2(
 // rms(rec)/rms(ion))) gives both channels the same RMS; a power of two keeps
 // the scaling exact (the centre test becomes Im >= s*Re, and Im/s is the
-// unscaled ion field bit for bit).  Sums in FP64.
+// unscaled ion field bit for bit).  Sums in FP64.  The first pass of a slice: it
+// empties the centre map (map, nullable) as well, a launch less (64^3: 5 of 110
+// us; 512^3: 0.08 ms of fill under the reads).
 // ------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_balance_partial(long n3, const float* __restrict__ a,
                                                          const float* __restrict__ b,
                                                          const float* __restrict__ c, CellConsts k,
-                                                         double* __restrict__ part) {
+                                                         double* __restrict__ part,
+                                                         int* __restrict__ map) {
   double sr = 0.0, si = 0.0;
   for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n3;
        i += (long)gridDim.x * blockDim.x) {
@@ -43,6 +46,7 @@ __global__ __launch_bounds__(256) void k_balance_partial(long n3, const float* _
     cell_fields(k, a, b, c, i, rec, ion, fr);
     sr += (double)rec * rec;
     si += (double)ion * ion;
+    if (map) map[i] = -1;
   }
   __shared__ double r1[256], r2[256];
   r1[threadIdx.x] = sr;
@@ -833,8 +837,13 @@ __host__ __device__ constexpr int dt_col_floats(int n) { return n + n / 8 + 1; }
 // QMAX >= a.q: the per-lane result array of the line pass.  The last tile
 // of a row may be partial (n a multiple of 8): its missing columns load as
 // empty (-1) lines and are not stored.
+// Bound by chains of dependent LDS reads: 8 waves a block keep the CU's wave slots
+// full (the LDS of the larger sides leaves room for 4 blocks), 4 left them half
+// empty: 512^3 0.70-0.77 -> 0.57-0.59 ms a pass, 600^3 1.6-1.7 -> 1.2-1.3; 16 were
+// slower from 96 up (512^3 0.66-0.71).  With one block or less per CU (up to 64) a wave per
+// column: 64^3 11-12 -> 8 us (8 waves: 9).
 template <int QMAX>
-__global__ __launch_bounds__(256) void k_dt_tile(DtArgs a, int axis, const int* in, int* out) {
+__global__ __launch_bounds__(1024) void k_dt_tile(DtArgs a, int axis, const int* in, int* out) {
   extern __shared__ int sm[];
   const int n = a.n, Q = a.q, cs = dt_col_floats(n);
   const int ntile = (n + kDtCols - 1) / kDtCols;
@@ -961,9 +970,9 @@ int balance_partials_count(long n3) {
 }
 
 void launch_balance(long n3, const float* a, const float* b, const float* c, CellConsts k,
-                    double* part, float* scale, hipStream_t s) {
+                    double* part, float* scale, int* map, hipStream_t s) {
   const int nb = balance_partials_count(n3);
-  hipLaunchKernelGGL(k_balance_partial, dim3(nb), dim3(256), 0, s, n3, a, b, c, k, part);
+  hipLaunchKernelGGL(k_balance_partial, dim3(nb), dim3(256), 0, s, n3, a, b, c, k, part, map);
   hipLaunchKernelGGL(k_balance_final, dim3(1), dim3(256), 0, s, part, nb, scale);
 }
 
@@ -1162,19 +1171,21 @@ int dt_q(int n) {
   return 0;
 }
 
+static unsigned dt_threads(unsigned blocks) { return blocks <= 256 ? 64 * kDtCols : 512; }
+
 void launch_dt_rows(const DtArgs& a, const int* in, int* out, hipStream_t s) {
   // axis i: tiles (j, p-block)
   const size_t lds = sizeof(int) * kDtCols * dt_col_floats(a.n);
   const dim3 g((unsigned)(a.n * ((a.n + kDtCols - 1) / kDtCols)));
-  if (a.q <= 8) hipLaunchKernelGGL(k_dt_tile<8>, g, dim3(256), lds, s, a, 1, in, out);
-  else hipLaunchKernelGGL(k_dt_tile<16>, g, dim3(256), lds, s, a, 1, in, out);
+  if (a.q <= 8) hipLaunchKernelGGL(k_dt_tile<8>, g, dim3(dt_threads(g.x)), lds, s, a, 1, in, out);
+  else hipLaunchKernelGGL(k_dt_tile<16>, g, dim3(dt_threads(g.x)), lds, s, a, 1, in, out);
 }
 void launch_dt_cols(const DtArgs& a, const int* in, int* out, hipStream_t s) {
   // axis j: tiles (i, p-block)
   const size_t lds = sizeof(int) * kDtCols * dt_col_floats(a.n);
   const dim3 g((unsigned)(a.n * ((a.n + kDtCols - 1) / kDtCols)));
-  if (a.q <= 8) hipLaunchKernelGGL(k_dt_tile<8>, g, dim3(256), lds, s, a, 0, in, out);
-  else hipLaunchKernelGGL(k_dt_tile<16>, g, dim3(256), lds, s, a, 0, in, out);
+  if (a.q <= 8) hipLaunchKernelGGL(k_dt_tile<8>, g, dim3(dt_threads(g.x)), lds, s, a, 0, in, out);
+  else hipLaunchKernelGGL(k_dt_tile<16>, g, dim3(dt_threads(g.x)), lds, s, a, 0, in, out);
 }
 void launch_dt_final(const DtArgs& a, const int* in, const float* pa, const float* pb,
                      const float* pc, CellConsts k, float* xhii, double* partials,

@@ -320,11 +320,10 @@ void enqueue_generic(sf21_hii_ctx* c, const float* a, const float* b, const floa
   hipStream_t s = c->stream;
   const GenPlan& g = c->gplan;
   const float2 none = make_float2(0.f, 0.f);
-  launch(c, "balance", [&] { launch_balance(n3, a, b, cc, k, c->bal_part, c->bal, s); });
+  launch(c, "balance", [&] { launch_balance(n3, a, b, cc, k, c->bal_part, c->bal, c->wmap, s); });
   launch(c, "gen_pack", [&] { launch_gen_pack(n3, a, b, cc, k, c->bal, c->spec, s); });
   for (int axis = 0; axis < 3; ++axis)
     launch(c, "gen_fwd", [&] { launch_gen_pass(g, axis, -1, 0, c->spec, c->spec, c->tw, none, s); });
-  launch(c, "fill_map", [&] { launch_fill_i32(c->wmap, -1, n3, s); });
   const int r_lo = only_radius >= 0 ? only_radius : 0;
   const int r_hi = only_radius >= 0 ? only_radius + 1 : (int)c->radii.size();
   for (int re = r_hi; re > r_lo; re -= c->Kg) {
@@ -368,10 +367,9 @@ void enqueue_fused(sf21_hii_ctx* c, const float* a, const float* b, const float*
   const long n3 = c->n3;
   const CellConsts k = cell_consts(c, z);
   hipStream_t s = c->stream;
-  launch(c, "balance", [&] { launch_balance(n3, a, b, cc, k, c->bal_part, c->bal, s); });
+  launch(c, "balance", [&] { launch_balance(n3, a, b, cc, k, c->bal_part, c->bal, c->wmap, s); });
   launch(c, "fwd_rows", [&] { launch_fwd_rows(n, a, b, cc, k, c->bal, c->spec, c->tw, s); });
   launch(c, "cols_fwd_j", [&] { launch_cols(n, n, 0, -1, c->spec, c->spec, 1, 0, c->tw, s, 16, kColsStream); });
-  launch(c, "fill_map", [&] { launch_fill_i32(c->wmap, -1, n3, s); });
   // radius batches in ascending radius (from the end of the descending
   // ladder): each batch's ball bounds exceed the earlier batches', which the
   // centre-map update relies on
@@ -681,7 +679,7 @@ void enqueue_diff_backward(sf21_hii_ctx* c, const float* g, const float* emis, d
   const CellConsts k = cell_consts(c, 0.0);  // direct inputs
   enqueue_diff_fields(c, g, emis, zeta);
   // forward spectrum Z of rec + i s ion, (p,j)-space
-  launch(c, "balance", [&] { launch_balance(n3, c->df_rec, c->df_ion, nullptr, k, c->bal_part, c->bal, s); });
+  launch(c, "balance", [&] { launch_balance(n3, c->df_rec, c->df_ion, nullptr, k, c->bal_part, c->bal, nullptr, s); });
   if (!kept) {
     launch(c, "fwd_rows", [&] { launch_fwd_rows(n, c->df_rec, c->df_ion, nullptr, k, c->bal, c->spec, c->tw, s); });
     launch(c, "cols_fwd_j", [&] { launch_cols(n, n, 0, -1, c->spec, c->spec, 1, 0, c->tw, s, 16, kColsStream); });
@@ -789,7 +787,7 @@ void enqueue_diff_backward_generic(sf21_hii_ctx* c, const float* g, const float*
   const float2 none = make_float2(0.f, 0.f);
   enqueue_diff_fields(c, g, emis, zeta);
   // forward spectrum Z of rec + i s ion
-  launch(c, "balance", [&] { launch_balance(n3, c->df_rec, c->df_ion, nullptr, k, c->bal_part, c->bal, s); });
+  launch(c, "balance", [&] { launch_balance(n3, c->df_rec, c->df_ion, nullptr, k, c->bal_part, c->bal, nullptr, s); });
   launch(c, "gen_pack", [&] { launch_gen_pack(n3, c->df_rec, c->df_ion, nullptr, k, c->bal, c->spec, s); });
   gen_fft3(c, c->spec, -1);
   // the real-space pair (N R_R, s N I_R) of radius r into ubuf
