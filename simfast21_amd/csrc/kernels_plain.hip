@@ -353,14 +353,34 @@ namespace sf21 {
 // half spectrum's.
 //
 // One wave per (i, j) row, lanes along p: |k|, and so the bin, never decreases
-// along a row, so the lanes of a bin are neighbours; a segmented wave sum
+// along a row, so the lanes of a bin are neighbours; a segmented sum
 // leaves each run's total in its first lane, which adds it to the block's FP64
 // sums in LDS.  GEO sums |k| and the mode count instead of |F|^2: they depend
-// on n and the bins only, and a context keeps them.  256^3: 0.58 -> 0.057 ms
-// (every mode added three LDS atomics to a few addresses, and one block then
-// read 2048 partials in turn).  Bound: the read of the spectrum.
+// on n and the bins only, and a context keeps them.  The sums stay within rows of
+// 16 lanes, where the neighbours' values come with the vector operation; over
+// the wave they cost 21 LDS permutes a chunk.  256^3: 0.58 ms (every mode added
+// three LDS atomics to a few addresses, and one block then read 2048 partials
+// in turn) -> 0.057 over the wave -> 0.038 ms.  Bound: the read of the spectrum.
 // ------------------------------------------------------------------------
 constexpr int kPkMaxBins = 64;
+
+template <int O>
+__device__ __forceinline__ double row_shl(double v) {
+  const int lo = __double2loint(v), hi = __double2hiint(v);
+  return __hiloint2double(__builtin_amdgcn_update_dpp(0, hi, 0x100 | O, 0xf, 0xf, false),
+                          __builtin_amdgcn_update_dpp(0, lo, 0x100 | O, 0xf, 0xf, false));
+}
+
+// One doubling step: the lane O above in the row of 16, if it has the same bin.
+template <int O, bool GEO>
+__device__ __forceinline__ void seg_add(int b, double& va, double& vb) {
+  const int ob = __builtin_amdgcn_update_dpp(-2, b, 0x100 | O, 0xf, 0xf, false);
+  const double oa = row_shl<O>(va), oc = GEO ? row_shl<O>(vb) : 0.0;
+  if (ob == b) {
+    va += oa;
+    if (GEO) vb += oc;
+  }
+}
 
 template <bool GEO>
 __global__ __launch_bounds__(256) void k_pk_partial(int n, const float2* __restrict__ spec,
@@ -392,18 +412,14 @@ __global__ __launch_bounds__(256) void k_pk_partial(int n, const float2* __restr
           va = (double)f.x * f.x + (double)f.y * f.y;
         }
       }
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int ob = __shfl_down(b, o, 64);
-        const double oa = __shfl_down(va, o, 64);
-        const double oc = GEO ? __shfl_down(vb, o, 64) : 0.0;
-        if (lane + o < 64 && ob == b) {
-          va += oa;
-          if (GEO) vb += oc;
-        }
+      if (h - q0 > 1) {  // the last element of a half row is alone
+        seg_add<1, GEO>(b, va, vb);
+        seg_add<2, GEO>(b, va, vb);
+        seg_add<4, GEO>(b, va, vb);
+        seg_add<8, GEO>(b, va, vb);
       }
-      const int prev = __shfl_up(b, 1, 64);
-      if (b >= 0 && (lane == 0 || prev != b)) {
+      const int prev = __builtin_amdgcn_update_dpp(-2, b, 0x111, 0xf, 0xf, false);  // row_shr:1
+      if (b >= 0 && prev != b) {
         atomicAdd(&s_a[b], va);
         if (GEO) atomicAdd(&s_b[b], vb);
       }
