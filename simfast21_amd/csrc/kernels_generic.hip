@@ -315,7 +315,8 @@ __global__ void k_gen_pack(long n3, const float* __restrict__ a, const float* __
 // lose more than the filter pass gains (28.2 + 40.0 + 25.4 ms against 35.1 +
 // 32.2 + 23.4).  Tried and slower: neighbouring tiles behind each other along
 // i in at most 40 groups (600^3 p pass 30.0 ms against 25.0); j blocks over
-// half the columns of a line (600^3 41.0 ms).
+// half the columns of a line (600^3 41.0 ms), or over its halves in turn with
+// both loaded first (43.9: 155 registers).
 // ------------------------------------------------------------------------
 #define SF21_GEN_SIDES(X)                                                                  \
   X(16) X(24) X(40) X(48) X(72) X(80) X(120) X(144) X(160) X(200) X(216) X(240) X(288) X(320) \

@@ -1086,9 +1086,8 @@ int create_deposit(const sf21_hii_config* cfg, sf21_hii_ctx** out) {
 
 // Entry points that need the transforms and the bubble finder's buffers.
 bool is_deposit(const sf21_hii_ctx* c) { return c && c->cfg.path == SF21_PATH_DEPOSIT; }
-// Sides without a register plan: the fused finder runs one radius per step
-// through the line passes; the autotuner searches their block order, and the
-// differentiable mode recomputes its fields there.
+// Sides without a register plan: the autotuner searches the line passes' block
+// order, and the differentiable mode recomputes its fields there.
 bool is_generic(const sf21_hii_ctx* c) { return c && c->generic; }
 
 // Autotuner on a side without a register plan: the XCD-order mask of the
@@ -1236,7 +1235,7 @@ int sf21_hii_create(const sf21_hii_config* cfg, sf21_hii_ctx** out) {
     c->Kd = 16;
   }
   if (c->K > (int)c->radii.size()) c->K = (int)c->radii.size();
-  if (c->generic) c->K = 1;  // one radius per step, in-kernel FP32 weights
+  if (c->generic) c->K = 1;  // reported; the batch is Kg, FP32 weights
   if (c->generic) c->filter_w = 1;
   if (c->Kd < 1 || c->Kd > c->K) c->Kd = c->K;
 
