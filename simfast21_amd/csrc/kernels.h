@@ -243,6 +243,8 @@ int sum_partials_count(long count);
 void launch_sum_f32(long count, const float* x, double* part, double* out, hipStream_t s);
 // allows the displacement deposit's LDS on the current device
 bool deposit_prepare();
+// the grid of -1 that the deposit adds to, then the deposit and its block average
+void launch_nldensity_start(int ng, float* grid, hipStream_t s);
 void launch_nldensity(int ng, int ns, int sm, const float* vx, const float* vy, const float* vz,
                       const float* delta0, float vscale, float growth_in, float growth,
                       float* grid, float* out, hipStream_t s);

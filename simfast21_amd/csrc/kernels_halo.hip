@@ -261,28 +261,49 @@ __global__ __launch_bounds__(kDepThreads) void k_displace_deposit(
   }
 }
 
-// Block average of sm^3 cells (compensated FP32 sum), then the scale.
-__global__ void k_smooth_scale(int ng, int ns, int sm, const float* __restrict__ grid,
-                               float scale, float* __restrict__ out) {
-  const long n3 = (long)ns * ns * ns;
+// Block average of sm^3 cells (compensated FP32 sum in the cells' order).  A
+// row of 64 lanes per row of blocks; PAIR: blocks of 2 on an even, aligned
+// grid, whose four pairs are loaded together.  Bound: the read of the grid.
+// 512^3 to 256^3: 0.157 ms with a 64-bit division per block and single loads,
+// 0.113 ms this way.
+template <bool PAIR>
+__global__ __launch_bounds__(256) void k_smooth_scale(int ng, int ns, int sm,
+                                                      const float* __restrict__ grid,
+                                                      float* __restrict__ out) {
   const float inv = 1.0f / ((float)sm * sm * sm);
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n3;
-       i += (long)gridDim.x * blockDim.x) {
-    const int a = (int)(i / ((long)ns * ns)), b = (int)((i / ns) % ns), c = (int)(i % ns);
-    float s = 0.0f, comp = 0.0f;
-    for (int u = 0; u < sm; ++u)
-      for (int v = 0; v < sm; ++v) {
-        const float* __restrict__ row = grid + ((long)(a * sm + u) * ng + (b * sm + v)) * ng + c * sm;
-        for (int w = 0; w < sm; ++w) {
-          const float yv = row[w] - comp;
-          const float t = s + yv;
-          comp = (t - s) - yv;
-          s = t;
+  for (int row = blockIdx.x * 4 + threadIdx.y; row < ns * ns; row += gridDim.x * 4) {
+    const int a = row / ns, b = row % ns;
+    const float* __restrict__ first = grid + ((long)a * sm * ng + (long)b * sm) * ng;
+    for (int c = threadIdx.x; c < ns; c += 64) {
+      float s = 0.0f, comp = 0.0f;
+      auto add = [&](float x) {
+        const float yv = x - comp;
+        const float t = s + yv;
+        comp = (t - s) - yv;
+        s = t;
+      };
+      if constexpr (PAIR) {
+        float2 x[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          x[q] = reinterpret_cast<const float2*>(first + ((long)(q >> 1) * ng + (q & 1)) * ng)[c];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          add(x[q].x);
+          add(x[q].y);
         }
+      } else {
+        for (int u = 0; u < sm; ++u)
+          for (int v = 0; v < sm; ++v) {
+            const float* __restrict__ line = first + ((long)u * ng + v) * ng + (long)c * sm;
+            for (int w = 0; w < sm; ++w) add(line[w]);
+          }
       }
-    out[i] = (s * inv) * scale;
+      out[(long)row * ns + c] = s * inv;
+    }
   }
 }
+
 
 template <class T>
 __global__ void k_zero(T* __restrict__ p, long count) {
@@ -350,19 +371,25 @@ bool deposit_prepare() {
                              (int)sizeof(double) * kDepCap) == hipSuccess;
 }
 
+void launch_nldensity_start(int ng, float* grid, hipStream_t s) {
+  const long g3 = (long)ng * ng * ng;
+  hipLaunchKernelGGL(k_fill_value, dim3(blocks_for(g3)), dim3(256), 0, s, grid, -1.0f, g3);
+}
+
 void launch_nldensity(int ng, int ns, int sm, const float* vx, const float* vy, const float* vz,
                       const float* delta0, float vscale, float growth_in, float growth,
                       float* grid, float* out, hipStream_t s) {
-  const long g3 = (long)ng * ng * ng;
   const long tiles = (long)((ng + kDepTX - 1) / kDepTX) * ((ng + kDepTY - 1) / kDepTY) *
                      ((ng + kDepTZ - 1) / kDepTZ);
-  hipLaunchKernelGGL(k_fill_value, dim3(blocks_for(g3)), dim3(256), 0, s, grid, -1.0f, g3);
   hipLaunchKernelGGL(k_displace_deposit, dim3((unsigned)(tiles < kDepBlocks ? tiles : kDepBlocks)),
                      dim3(kDepThreads), sizeof(double) * kDepCap, s, ng, (int)tiles, vx, vy, vz,
                      delta0, vscale, growth_in, growth, grid);
-  if (out)
-    hipLaunchKernelGGL(k_smooth_scale, dim3(blocks_for((long)ns * ns * ns)), dim3(256), 0, s, ng,
-                       ns, sm, grid, 1.0f, out);
+  if (!out) return;
+  const dim3 g(blocks_for((long)ns * ns * 64)), b(64, 4);
+  if (sm == 2 && ng % 2 == 0 && reinterpret_cast<uintptr_t>(grid) % sizeof(float2) == 0)
+    hipLaunchKernelGGL(k_smooth_scale<true>, g, b, 0, s, ng, ns, sm, grid, out);
+  else
+    hipLaunchKernelGGL(k_smooth_scale<false>, g, b, 0, s, ng, ns, sm, grid, out);
 }
 
 void launch_halo_emissivity(long nhalos, const float* halos, int ng, int ns, int sm, float k_rion,

@@ -2088,8 +2088,9 @@ int sf21_nldensity_dev(sf21_hii_ctx* c, const sf21_params* p, double z, const fl
   // Mpc/h, the files in Mpc), the z = 0 mass 1 + delta0 D(300), the
   // displacement factor D(z) - D(300)
   if (!deposit_prepare()) return SF21_ERR_HIP;
+  launch(c, "nldensity_start", [&] { launch_nldensity_start(ng, grid, c->stream); });
   const double zs[2] = {300.0, z};
-  double gs[2];
+  double gs[2];  // while the grid is filled
   sf21_growth_many(p, 2, zs, gs);
   const double growth_in = gs[0], growth = gs[1] - growth_in;
   const double vscale = (double)ng / p->box_len * p->hubble;

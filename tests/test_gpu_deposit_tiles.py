@@ -63,3 +63,30 @@ def test_displacement_of_many_tiles(torch_cuda, m, amp, shift):
         got = box.cpu().numpy().reshape(m, m, m)
         assert np.abs(got - ref).max() <= tol, (rep, np.abs(got - ref).max(), tol)
     ctx.close()
+
+
+@pytest.mark.parametrize("n,m,offset", [(20, 40, 0), (20, 40, 1), (20, 41, 0), (7, 24, 0), (33, 67, 1),
+                                        (70, 140, 0), (70, 70, 0)])
+def test_block_average(torch_cuda, n, m, offset):
+    """The averages against the same compensated FP32 sums in numpy, exactly:
+    blocks of 1 to 3 cells, even and odd grids, a grid off its alignment."""
+    torch = torch_cuda
+    torch.manual_seed(m)
+    p = dict(hubble=H, omega_m=OM, omega_b=0.045, omega_lambda=OL, box_len=1.0 * m, n=n, n_halo=m)
+    v = [20 * torch.randn(m ** 3, device="cuda") for _ in range(3)]
+    ctx = sf.HiiContext(n, 1.0 * m, [], sf.INPUT_HALO, sf.PATH_DEPOSIT, n_halo=m)
+    box = torch.empty(m ** 3 + 1, device="cuda")[offset:offset + m ** 3]
+    out, _ = ctx.nldensity(p, 9.0, *v, torch.randn(m ** 3, device="cuda"), box_halo=box)
+    ctx.close()
+    g = box.cpu().numpy().reshape(m, m, m)
+    sm = int(np.floor(np.float32(m) / n + 0.5))
+    sm -= 1 if n * sm > m else 0
+    total = np.zeros((n, n, n), np.float32)
+    comp = np.zeros_like(total)
+    for a, b, c in np.ndindex(sm, sm, sm):
+        y = g[a:n * sm:sm, b:n * sm:sm, c:n * sm:sm] - comp
+        t = total + y
+        comp = (t - total) - y
+        total = t
+    ref = total * (np.float32(1) / (np.float32(sm) * sm * sm))
+    assert np.array_equal(out.cpu().numpy().reshape(n, n, n), ref)
