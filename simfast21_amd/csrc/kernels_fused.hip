@@ -1119,13 +1119,36 @@ bool plane_prepare(int n) {
   return ok;
 }
 
+// Radii per block of the plane pass.  Where one block fills a CU's LDS (96 and
+// 128): the split whose rounds of 256 blocks walk the fewest radii, a block's
+// start counted as one more (96^3, 31 radii: 8 groups, 3 rounds of 4 radii,
+// 0.109 ms; 4 groups, 2 rounds of 8, the second half full, 0.137).  Smaller
+// planes share the CU: enough groups for 16 waves (64^3 0.0205 ms, 0.0213 with
+// every block resident at once).
+static int plane_radii(int planes, int waves, int lds, int nrad) {
+  if (163840 / lds > 1) {
+    const int g = radius_groups((long)planes * waves, nrad);
+    return (nrad + g - 1) / g;
+  }
+  int best = nrad;
+  long cost = LONG_MAX;
+  for (int per = nrad; per >= 1; --per) {
+    const long blocks = (long)planes * ((nrad + per - 1) / per);
+    const long c = (blocks + 255) / 256 * (per + 1);
+    if (c < cost) {
+      cost = c;
+      best = per;
+    }
+  }
+  return best;
+}
+
 void launch_plane_crit(int n, const float2* u, int nrad, long ustride, const int* d2max,
                        const float* bal, int* wmap, float2* dbg, float2* keep, const float2* tw,
                        hipStream_t s) {
 #define X(L)                                                                              \
   if (n == L) {                                                                           \
-    const int g = radius_groups((long)L * ((PlaneCfg<L>::kThreads + 63) / 64), nrad);     \
-    const int per = (nrad + g - 1) / g;                                                   \
+    const int per = plane_radii(L, (PlaneCfg<L>::kThreads + 63) / 64, PlaneCfg<L>::kLds, nrad); \
     hipLaunchKernelGGL(k_plane_crit<L>, dim3(L, (nrad + per - 1) / per),                  \
                        dim3(PlaneCfg<L>::kThreads), PlaneCfg<L>::kLds, s, u, \
                        nrad, per, ustride, d2max, bal, wmap, dbg, keep, tw);              \

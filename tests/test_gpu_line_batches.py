@@ -39,7 +39,10 @@ def centre_map(n, side, radii, a, b, stats=None):
     return w
 
 
-@pytest.mark.parametrize("n,nr", [(24, 9), (120, 11), (144, 7), (200, 7), (576, 14)])
+# 64, 96 and 128 have a plan: their plane pass splits a ladder over blocks by
+# the room in LDS (one block a CU at 96 and 128)
+@pytest.mark.parametrize("n,nr", [(24, 9), (120, 11), (144, 7), (200, 7), (576, 14),
+                                  (64, 27), (96, 31), (96, 2), (128, 9)])
 def test_ladder_equals_its_parts(torch_cuda, n, nr):
     side = 1.5 * n
     radii = list(np.geomspace(0.25 * side, 2.0, nr))
