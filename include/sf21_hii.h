@@ -130,16 +130,18 @@ int sf21_hii_run_multi_dev(int nbox, sf21_hii_ctx *const *ctx, const float *cons
  * in N_halo cell units (auxiliary.h:13-17, output_files.txt:10-14).
  * Emissivity box = smooth_box(CIC(Rion(M, z))) * (dx_s/dx_h)^3 * fesc
  * (get_HIIbubbles.c:233-259); _dev takes device pointers.  run_slice_halo
- * takes host delta and catalog and runs the whole slice. */
+ * takes host delta and catalog and runs the whole slice.  The deposit adds
+ * in FP64 (n^3 doubles, allocated with the first call; SF21_ERR_ALLOC if they
+ * do not fit), in FP32 where an n-block is one cell. */
 int sf21_hii_halo_emissivity_dev(sf21_hii_ctx *ctx, const float *halos, long n_halos, double z,
                                  float *ion_out);
 /* Allocation-free variant of sf21_hii_halo_emissivity_dev: no counterpart
  * in the reference; it is for callers that cannot allocate device memory
  * (code under hipGraph capture, serving loops, harnesses that forbid
  * hipMalloc).  Same arguments and result (the same kernels); the n^3 FP64
- * sums live in a buffer that the context allocates when it is created (for
- * input_mode SF21_INPUT_HALO and N_halo <= 256; larger grids ->
- * SF21_ERR_ARG).  Enqueued on the context's stream without host
+ * sums live in a buffer that the context allocates when it is created
+ * (sf21_hii_create fails if it cannot; for input_mode SF21_INPUT_HALO and
+ * N_halo <= 256, larger grids -> SF21_ERR_ARG).  Enqueued on the context's stream without host
  * synchronisation. */
 int sf21_hii_halo_emissivity_noalloc(sf21_hii_ctx *ctx, const float *halos, long n_halos,
                                      double z, float *ion_out);
@@ -174,7 +176,8 @@ int sf21_t21_dev(sf21_hii_ctx *ctx, const sf21_params *p, double z, const float 
  * SFRD box of one redshift from a halo catalog (get_SFR.c:98-148; device
  * pointers): CIC of sfr(M, z) = Rion(M, z)/Qion(z) (user_functions.c:71-74)
  * on the N_halo^3 grid, smooth_box to n^3, divided by dx_halo^3 (Msun per
- * year per (Mpc/h)^3).  The context needs n_halo >= n.  *mean (nullable):
+ * year per (Mpc/h)^3).  The context needs n_halo >= n; sums as in
+ * sf21_hii_halo_emissivity_dev.  *mean (nullable):
  * the box average in FP64 (the sfrd_av table). */
 int sf21_sfrd_dev(sf21_hii_ctx *ctx, const float *halos, long n_halos, double z, float *out,
                   double *mean);

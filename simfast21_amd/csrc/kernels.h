@@ -248,7 +248,7 @@ void launch_nldensity_start(int ng, float* grid, hipStream_t s);
 void launch_nldensity(int ng, int ns, int sm, const float* vx, const float* vy, const float* vz,
                       const float* delta0, float vscale, float growth_in, float growth,
                       float* grid, float* out, hipStream_t s);
-// acc: n^3 doubles to accumulate in; null: FP32 sums in out
+// acc: ns^3 doubles to accumulate in (unused with sm = 1: FP32 sums in out)
 void launch_halo_emissivity(long nhalos, const float* halos, int ng, int ns, int sm, float k_rion,
                             float c2, float c3, float scale, double* acc, float* out,
                             hipStream_t s);

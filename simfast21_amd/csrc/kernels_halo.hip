@@ -398,8 +398,7 @@ void launch_halo_emissivity(long nhalos, const float* halos, int ng, int ns, int
   const long n3 = (long)ns * ns * ns;
   const float f = (float)((double)scale / ((double)sm * sm * sm));
   const dim3 g(blocks_for(n3)), gh(blocks_for(nhalos)), b(256);
-  if (sm == 1) acc = nullptr;  // a block is one cell: the deposit's own FP32 sums
-  if (!acc) {
+  if (sm == 1) {  // a block is one cell: the deposit's own FP32 sums
     hipLaunchKernelGGL(k_zero<float>, g, b, 0, s, out, n3);
     if (nhalos > 0)
       hipLaunchKernelGGL(k_cic_rion<float>, gh, b, 0, s, nhalos, halos, ng, ns, sm, k_rion, c2, c3,

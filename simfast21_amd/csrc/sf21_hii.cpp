@@ -1041,11 +1041,19 @@ void apply_choice(sf21_hii_ctx* c, const TuneChoice& t) {
 // Largest N_halo^3 that sf21_hii_halo_emissivity_noalloc takes (N_halo <= 256).
 constexpr long kNoAllocGrid = 1L << 24;
 
-// FP64 sums of the catalog deposits; left null (FP32 sums in the output box)
-// where they do not fit.  Contexts that sf21_hii_halo_emissivity_noalloc takes
-// allocate them when they are created.
-void ensure_halo_acc(sf21_hii_ctx* c) {
-  if (!c->halo_acc) (void)dev_alloc(&c->halo_acc, (size_t)c->n3);
+// smooth_box's block size (auxiliary.c:654-656)
+long smooth_block(int ng, int ns) {
+  long sm = (long)roundf((1.0f * ng) / ns);
+  if ((long)ns * sm > ng) sm--;
+  return sm;
+}
+
+// FP64 sums of the catalog deposits (blocks of one cell add in FP32, as a
+// deposit on that cell does, and need none).  Contexts that
+// sf21_hii_halo_emissivity_noalloc takes allocate them when they are created.
+int ensure_halo_acc(sf21_hii_ctx* c) {
+  if (c->halo_acc || smooth_block(c->cfg.n_halo, c->n) <= 1) return SF21_OK;
+  return dev_alloc(&c->halo_acc, (size_t)c->n3);
 }
 bool noalloc_context(const sf21_hii_ctx* c) {
   const long ng = c->cfg.n_halo;
@@ -1079,7 +1087,14 @@ int create_deposit(const sf21_hii_config* cfg, sf21_hii_ctx** out) {
     return SF21_ERR_HIP;
   }
   c->own_stream = true;
-  if (noalloc_context(c)) ensure_halo_acc(c);
+  if (noalloc_context(c)) {
+    const int rc = ensure_halo_acc(c);
+    if (rc) {
+      free_all(c);
+      delete c;
+      return rc;
+    }
+  }
   *out = c;
   return SF21_OK;
 }
@@ -1351,7 +1366,7 @@ int sf21_hii_create(const sf21_hii_config* cfg, sf21_hii_ctx** out) {
         (rc = dev_alloc(&c->flag_dev, 1)))
       goto fail;
   }
-  if (noalloc_context(c)) ensure_halo_acc(c);
+  if (noalloc_context(c) && (rc = ensure_halo_acc(c))) goto fail;
   // the tables are complete before any other stream can use them
   if (hipStreamSynchronize(c->stream) != hipSuccess || (rc = check_hip())) {
     if (!rc) rc = SF21_ERR_HIP;
@@ -1860,19 +1875,17 @@ int sf21_hii_power_spectrum_dev(sf21_hii_ctx* c, const float* field, int nbins, 
 }  // extern "C"
 
 namespace {
-// Launch constants of the halo-mode emissivity: smooth_box's block size
-// (auxiliary.c:654-656), the volume ratio times fesc (get_HIIbubbles.c:253-258)
+// Launch constants of the halo-mode emissivity: smooth_box's block size, the
+// volume ratio times fesc (get_HIIbubbles.c:253-258)
 // and Rion's redshift factor (user_functions.c:40-47: c1 (1+z)^c4 / V_norm).
 struct HaloConsts {
   long sm;
   float scale, k_rion;
 };
 int halo_consts(const sf21_hii_ctx* c, double z, HaloConsts* k) {
-  const int ng = c->cfg.n_halo, ns = c->n;
-  k->sm = (long)roundf((1.0f * ng) / ns);
-  if ((long)ns * k->sm > ng) k->sm--;
+  k->sm = smooth_block(c->cfg.n_halo, c->n);
   if (k->sm < 1) return SF21_ERR_ARG;
-  const double dx_h = c->L / ng;
+  const double dx_h = c->L / c->cfg.n_halo;
   k->scale = (float)(std::pow(c->dx / dx_h, 3) * c->cfg.fesc);
   k->k_rion = (float)(1.575e39 * std::pow(1.0 + z, 2.27044695e+00) / kVnorm);
   return SF21_OK;
@@ -1890,7 +1903,8 @@ int sf21_hii_halo_emissivity_dev(sf21_hii_ctx* c, const float* halos, long nhalo
   if (halo_consts(c, z, &k)) return SF21_ERR_ARG;
   if (hipSetDevice(c->cfg.device) != hipSuccess) return SF21_ERR_HIP;
   (void)hipGetLastError();
-  ensure_halo_acc(c);
+  const int rc = ensure_halo_acc(c);
+  if (rc) return rc;
   launch(c, "halo_emissivity", [&] {
     launch_halo_emissivity(nhalos, halos, c->cfg.n_halo, c->n, (int)k.sm, k.k_rion,
                            (float)9.367608e+07, 0.44f, k.scale, c->halo_acc, ion_out, c->stream);
@@ -2013,12 +2027,6 @@ int sf21_t21_dev(sf21_hii_ctx* c, const sf21_params* p, double z, const float* d
 
 // ---- the step before: SFRD and non-linear density deposits --------------
 namespace {
-// smooth_box's block size (auxiliary.c:654-656)
-long smooth_block(int ng, int ns) {
-  long sm = (long)roundf((1.0f * ng) / ns);
-  if ((long)ns * sm > ng) sm--;
-  return sm;
-}
 int ensure_halo_grid(sf21_hii_ctx* c) {
   const long ng = c->cfg.n_halo;
   if (c->halo_grid) return SF21_OK;
@@ -2052,7 +2060,7 @@ int sf21_sfrd_dev(sf21_hii_ctx* c, const float* halos, long nhalos, double z, fl
   const int ng = c->cfg.n_halo, ns = c->n;
   const long sm = smooth_block(ng, ns);
   if (sm < 1) return SF21_ERR_ARG;
-  ensure_halo_acc(c);
+  if ((rc = ensure_halo_acc(c))) return rc;
   const double dx_h = c->L / ng;
   // sfr = Rion/Qion (user_functions.c:71-74); Msun/yr per halo, then the
   // block average divided by dx_halo^3 (get_SFR.c:126-139)
