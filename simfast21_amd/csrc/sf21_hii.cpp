@@ -1295,7 +1295,7 @@ int sf21_hii_create(const sf21_hii_config* cfg, sf21_hii_ctx** out) {
       rc = SF21_ERR_HIP;
       goto fail;
     }
-    if (c->filter_w) {
+    if (c->filter_w && cfg->path == SF21_PATH_FUSED) {
       // the FP32 weight table, if it takes at most 1/16 of the free memory
       // (otherwise the filter pass evaluates the weights; generic sides fill a
       // table of one batch, at most 16 GiB of pairs, before each batch)
