@@ -83,11 +83,13 @@ typedef struct sf21_hii_config {
   int device;            /* HIP device ordinal */
   int filter_tile;       /* columns per block of the fused filter pass: 4, 8, 16 or 0 (auto) */
   int filter_w;          /* top-hat weights W(|k| R): 0 = automatic (FP32),
-                            1 = FP32 evaluation (series below |k|R = 1.25,
-                            3 (sin x - x cos x)/x^3 above; kept in a table per context
-                            while it takes at most 1/16 of the free device memory), 2 = FP64 table per integer
-                            |k|^2 rounded to float (sides without a register plan always
-                            evaluate in the kernel) */
+                            1 = FP32 (series below |k|R = 1.25, 3 (sin x - x cos x)/x^3
+                            above), read from a table: n^3/4 floats per radius, the
+                            whole ladder where that takes at most 1/16 of the free
+                            device memory, else a share of it refilled before each
+                            filter pass, with the same values; 2 = FP64 table per
+                            integer |k|^2 rounded to float (sides without a register
+                            plan have the FP32 table only) */
   int n_halo;            /* N_halo, halo mode: the catalog grid (>= n) */
 } sf21_hii_config;
 
@@ -291,8 +293,8 @@ int sf21_hii_filtered_dev(sf21_hii_ctx *ctx, const float *a, const float *b, con
  * changes launch shapes or block order only: the results are identical. */
 int sf21_hii_autotune(sf21_hii_ctx *ctx, const float *a, const float *b, const float *c,
                       double z, const char *cache_path, double *best_ms);
-/* Current choices: filter tile, radius batch, top-hat weights (1 in the
- * kernel, 2 table), column-pass tile, column-pass variant (bit 0: 16 values
+/* Current choices: filter tile, radius batch, top-hat weights (1 FP32, 2
+ * from FP64), column-pass tile, column-pass variant (bit 0: 16 values
  * per thread, bit 1: prefetching blocks), 16 values per thread in the
  * centre-test pass (0/1), filter blocks over mirror pairs of i-lines that
  * share the weights (0/1); any pointer may be NULL. */

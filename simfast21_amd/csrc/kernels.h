@@ -79,28 +79,25 @@ void launch_fwd_rows(int n, const float* a, const float* b, const float* c, Cell
 void launch_cols(int n, int width, int axis, int sign, const float2* in, float2* out,
                  int nbatch, long bstride, const float2* tw, hipStream_t s, int tile = 16,
                  int variant = 0);
-// Top-hat weights of the filter passes, all radii of the ladder.  mode 0:
-// lut, the FP64 table per integer |k|^2 (mlut entries per radius); mode 1:
-// FP32, from the weight table or, without one, evaluated in the pass from
-// kappa = dk R as hi + lo.
+// Top-hat weights of a filter pass, from its first radius on: lut (mlut entries
+// per radius), rounded from FP64 per integer |k|^2, or, with lut null, the FP32
+// weight table.
 struct FilterW {
-  int mode;
   const float* lut;
   long mlut;
   const float* table;
-  const float2* kappa;
 };
 // floats of one radius of the weight table: [fj][p/g][fi][p%g], g = 16, or 8
 // on sides that are an odd multiple of 8
 constexpr long wtab_radius(int n) { return (long)(n / 2 + 1) * (n / 2 + 1) * n; }
 void launch_w_table(int n, int nr, const float2* kappa, float* wt, hipStream_t s);
-// radii rb .. rb + nrad - 1 of the ladder; mirror: the block order that runs
-// the i-lines kj and n - kj, which share their weights, together on one XCD;
+// mirror: the block order that runs the i-lines kj and n - kj, which share their
+// weights, together on one XCD;
 // t16: u in the 16-column tile layout of launch_cols (the p pass then reads
 // it with t16 as well)
 void launch_filter_i(int n, const float2* spec, float2* u, int nrad, long ustride,
-                     const FilterW& w, int rb, const float2* tw, hipStream_t s, int tile,
-                     bool mirror = false, bool t16 = false);
+                     const FilterW& w, const float2* tw, hipStream_t s, int tile, bool mirror,
+                     bool t16);
 // sides whose j and p inverses and centre test run plane by plane (u in the
 // natural layout); prepare allows the blocks' LDS on the current device
 bool plane_side(int n);

@@ -282,9 +282,9 @@ __global__ __launch_bounds__(TILE*(L / E)) void k_cols_pipe(const float2* in, fl
 // Top-hat weights of every radius, laid out as the filter passes read them:
 // wt[r][fj][p/g][fi][p%g] (fj, fi <= n/2 the folded frequencies along j and i;
 // g = 16, or 8 on sides that are an odd multiple of 8): a block's weights of
-// one radius are one contiguous piece of whole cache lines.  The same function
-// of the same integer |k|^2 as an evaluation in the filter pass, so the same
-// values; computed once per context.
+// one radius are one contiguous piece of whole cache lines.  A function of the
+// integer |k|^2 alone, computed once per context (or, where the ladder's table
+// would take too much memory, a share of it before each filter pass).
 // ------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_w_table(int n, const float2* __restrict__ kappa,
                                                  float* __restrict__ wt) {
@@ -381,18 +381,15 @@ __global__ __launch_bounds__(TILE*(L / FilterE<L>::kE)) void k_filter_tab(
   }
 }
 
-// The filter pass without the weight table: weights from the FP64 table per
-// integer |k|^2 (WTAB), or evaluated per position (no memory for the
-// table).  One line per block.
-template <int L, int TILE, bool WTAB>
-__global__ __launch_bounds__(TILE*(L / Plan<L>::E)) void k_filter_i(
+// The filter pass with the FP64 weights per integer |k|^2 (a setting of the
+// configuration): one line per block.
+template <int L, int TILE>
+__global__ __launch_bounds__(TILE*(L / Plan<L>::E)) void k_filter_lut(
     const float2* __restrict__ spec, float2* __restrict__ u, int nrad, long ustride,
-    const float* __restrict__ wlut, long mlut, const float2* __restrict__ kappa,
-    const float2* __restrict__ tw, int t16) {
+    const float* __restrict__ wlut, long mlut, const float2* __restrict__ tw, int t16) {
   constexpr int E = Plan<L>::E, TPL = L / E, NT = L / TILE;
   __shared__ float lds[TILE * 2 * LdsLine<L>::kFloats];
-  // mirror pairs (t, TPL - t) in adjacent slots: lanes ^ TILE share W
-  const int c = threadIdx.x % TILE, t = paired_slot_to_t(threadIdx.x / TILE, TPL);
+  const int c = threadIdx.x % TILE, t = threadIdx.x / TILE;
   const int kj = blockIdx.x / NT;
   const int kp = (blockIdx.x % NT) * TILE + c;
   float* sre = lds + c * 2 * LdsLine<L>::kFloats;
@@ -404,28 +401,16 @@ __global__ __launch_bounds__(TILE*(L / Plan<L>::E)) void k_filter_i(
   for (int m = 0; m < E; ++m) z[m] = src[(t + TPL * m) * (L * L)];
   line_fft<L, -1>(z, sre, sim, t, tw);
   const int mjp = fold_sq(kj, L) + fold_sq(kp, L);
-  // |k|^2 and its square root for the lower-half positions (radius-independent)
-  int mm[E / 2 + 1];
-  SqrtPair sq[E / 2 + 1];
-#pragma unroll
-  for (int m = 0; m <= E / 2; ++m) {
-    mm[m] = mjp + fold_sq((t + TPL * m) % L, L);
-    sq[m] = sqrt_pair(mm[m]);
-  }
 #pragma unroll 1
   for (int r = 0; r < nrad; ++r) {
     const int tl = opaque_lane(t);
-    float wv[E];
-    if constexpr (WTAB) {
-      const float* __restrict__ w = wlut + (long)r * mlut;
-#pragma unroll
-      for (int m = 0; m < E; ++m) wv[m] = w[mjp + fold_sq(tl + TPL * m, L)];
-    } else {
-      w_line_shared<L, E, TILE>(kappa[r], sq, mm, t, wv);  // dk R as hi + lo
-    }
+    const float* __restrict__ w = wlut + (long)r * mlut;
     float2 v[E];
 #pragma unroll
-    for (int m = 0; m < E; ++m) v[m] = make_float2(z[m].x * wv[m], z[m].y * wv[m]);
+    for (int m = 0; m < E; ++m) {
+      const float wv = w[mjp + fold_sq(tl + TPL * m, L)];
+      v[m] = make_float2(z[m].x * wv, z[m].y * wv);
+    }
     line_fft<L, +1>(v, sre, sim, tl, tw);
     // t16: as k_filter_tab
     float2* __restrict__ dst =
@@ -1072,32 +1057,27 @@ void launch_w_table(int n, int nr, const float2* kappa, float* wt, hipStream_t s
 }
 
 void launch_filter_i(int n, const float2* spec, float2* u, int nrad, long ustride,
-                     const FilterW& w, int rb, const float2* tw, hipStream_t s, int tile, bool mirror,
+                     const FilterW& w, const float2* tw, hipStream_t s, int tile, bool mirror,
                      bool t16) {
   const int lay = t16 ? 1 : 0;
-  const float* wt = w.table ? w.table + rb * wtab_radius(n) : nullptr;
-  const float* lut = w.lut ? w.lut + (long)rb * w.mlut : nullptr;
 #define X(L, TL)                                                                          \
   if (n == L && tile == TL) {                                                             \
-    constexpr int NT = TL * (L / Plan<L>::E), CT = L / TL;                                \
-    if (w.mode == 0)                                                                      \
-      hipLaunchKernelGGL((k_filter_i<L, TL, true>), dim3(L * CT), dim3(NT), 0, s, spec, u, nrad, \
-                         ustride, lut, w.mlut, w.kappa + rb, tw, lay);                    \
-    else if (!wt)                                                                         \
-      hipLaunchKernelGGL((k_filter_i<L, TL, false>), dim3(L * CT), dim3(NT), 0, s, spec, u, nrad, \
-                         ustride, lut, w.mlut, w.kappa + rb, tw, lay);                    \
-    else {                                                                                \
-      constexpr int NTF = TL * (L / FilterE<L>::kE);                                      \
-      const int g = radius_groups((long)L * CT * ((NTF + 63) / 64), nrad);                \
+    constexpr int CT = L / TL;                                                            \
+    if (w.lut) {                                                                          \
+      hipLaunchKernelGGL((k_filter_lut<L, TL>), dim3(L * CT), dim3(TL * (L / Plan<L>::E)), 0, s, \
+                         spec, u, nrad, ustride, w.lut, w.mlut, tw, lay);                 \
+    } else {                                                                              \
+      constexpr int NT = TL * (L / FilterE<L>::kE);                                       \
+      const int g = radius_groups((long)L * CT * ((NT + 63) / 64), nrad);                 \
       const int per = (nrad + g - 1) / g;                                                 \
       const int mir = mirror && (L * CT) % 16 == 0;                                       \
-      hipLaunchKernelGGL((k_filter_tab<L, TL>), dim3(L * CT, (nrad + per - 1) / per), dim3(NTF), \
-                         0, s, spec, u, nrad, per, ustride, wt, tw, mir, lay);            \
+      hipLaunchKernelGGL((k_filter_tab<L, TL>), dim3(L * CT, (nrad + per - 1) / per), dim3(NT), \
+                         0, s, spec, u, nrad, per, ustride, w.table, tw, mir, lay);       \
     }                                                                                     \
     return;                                                                               \
   }
 #define Y(L) X(L, 4) X(L, 8) X(L, 16)
-  Y(32) Y(64) Y(96) Y(128) Y(192) Y(256) Y(512)
+  SF21_SIZES(Y)
 #undef Y
 #undef X
 }

@@ -129,7 +129,7 @@ struct sf21_hii_ctx {
   float* wlut = nullptr;
   long mlut = 0;
   float* wtab = nullptr;  // FP32 top-hat weights per radius (wtab_radius floats each)
-  bool wtab_all = false;  // wtab holds every radius (else one batch, filled per batch)
+  int Kw = 0;  // radii that wtab holds: the ladder, or a share refilled before each filter pass
   int Kg = 1;             // generic sides: radii per batch
   bool plane = false;     // j and p inverses and centre test plane by plane
   int* d_d2 = nullptr;
@@ -308,6 +308,29 @@ int check_hip() {
   return e == hipSuccess ? SF21_OK : SF21_ERR_HIP;
 }
 
+// The filter pass of the radii rb .. rb + kk - 1 into ubuf; t16 as launch_filter_i.
+// Where the weight table does not hold the whole ladder it is refilled, and the
+// pass runs, for as many radii at a time as it holds.
+void enqueue_filter(sf21_hii_ctx* c, int rb, int kk, bool t16) {
+  hipStream_t s = c->stream;
+  const bool refill = c->filter_w && c->Kw < (int)c->radii.size();
+  const int step = refill ? std::min(kk, c->Kw) : kk;
+  for (int q = 0; q < kk; q += step) {
+    const int r = rb + q, m = std::min(step, kk - q);
+    float2* u = c->ubuf + (long)q * c->n3;
+    if (refill)
+      launch(c, "w_table", [&] { launch_w_table(c->n, m, c->d_kappa + r, c->wtab, s); });
+    const FilterW w{c->filter_w ? nullptr : c->wlut + (long)r * c->mlut, c->mlut,
+                    c->wtab + (refill ? 0 : r * wtab_radius(c->n))};
+    if (c->generic)
+      launch(c, "gen_filter_i", [&] { launch_gen_filter(c->gplan, c->spec, u, m, w.table, c->tw, s); });
+    else
+      launch(c, "filter_i", [&] {
+        launch_filter_i(c->n, c->spec, u, m, c->n3, w, c->tw, s, c->tile_filter, c->filter_pair, t16);
+      });
+  }
+}
+
 // ---- fused exact path on a generic side ---------------------------------
 // Forward transforms of z = rec + i s ion along p, j, i; per batch of Kg radii
 // in ascending order, the filtered inverse along i, the inverse along j and
@@ -329,10 +352,7 @@ void enqueue_generic(sf21_hii_ctx* c, const float* a, const float* b, const floa
   for (int re = r_hi; re > r_lo; re -= c->Kg) {
     const int rb = std::max(r_lo, re - c->Kg);
     const int kk = re - rb;
-    const float* wt = c->wtab + (c->wtab_all ? rb * wtab_radius(c->n) : 0);
-    if (!c->wtab_all)
-      launch(c, "w_table", [&] { launch_w_table(c->n, kk, c->d_kappa + rb, c->wtab, s); });
-    launch(c, "gen_filter_i", [&] { launch_gen_filter(g, c->spec, c->ubuf, kk, wt, c->tw, s); });
+    enqueue_filter(c, rb, kk, false);
     if (!gen_plane_side(c->n))
       launch(c, "gen_inv_j", [&] { launch_gen_inv_j(g, c->ubuf, kk, c->tw, s); });
     launch(c, "gen_inv_p_crit", [&] {
@@ -348,10 +368,6 @@ void enqueue_generic(sf21_hii_ctx* c, const float* a, const float* b, const floa
   launch(c, "sum", [&] {
     launch_sum_partials(c->partials, c->npart, 1.0 / (double)n3, neutral_slot, s);
   });
-}
-
-FilterW filter_weights(const sf21_hii_ctx* c) {
-  return FilterW{c->filter_w, c->wlut, c->mlut, c->wtab, c->d_kappa};
 }
 
 // ---- fused exact path: enqueue one slice -------------------------------
@@ -378,10 +394,7 @@ void enqueue_fused(sf21_hii_ctx* c, const float* a, const float* b, const float*
   for (int re = r_hi; re > r_lo; re -= c->K) {
     const int rb = std::max(r_lo, re - c->K);
     const int kk = re - rb;
-    launch(c, "filter_i", [&] {
-      launch_filter_i(n, c->spec, c->ubuf, kk, n3, filter_weights(c), rb, c->tw, s, c->tile_filter,
-                      c->filter_pair, !c->plane);
-    });
+    enqueue_filter(c, rb, kk, !c->plane);
     if (c->plane) {
       launch(c, "plane_crit", [&] {
         launch_plane_crit(n, c->ubuf, kk, n3, c->d_d2 + rb, c->bal, c->wmap, dbg,
@@ -695,10 +708,7 @@ void enqueue_diff_backward(sf21_hii_ctx* c, const float* g, const float* emis, d
                         n3, s, true);
       });
     } else {
-      launch(c, "filter_i", [&] {
-        launch_filter_i(n, c->spec, c->ubuf, kk, n3, filter_weights(c), rb, c->tw, s, c->tile_filter,
-                        c->filter_pair);
-      });
+      enqueue_filter(c, rb, kk, false);
       launch(c, "cols_inv_j", [&] { launch_cols(n, n, 0, +1, c->ubuf, c->ubuf, kk, n3, c->tw, s, c->cols_tile, c->cols_wide | kColsStream); });
       launch(c, "rows_phi", [&] {
         launch_rows_phi(n, c->ubuf, kk, n3, c->bal, c->df_st, inv_tau, c->tw,
@@ -744,10 +754,7 @@ void enqueue_diff_backward(sf21_hii_ctx* c, const float* g, const float* emis, d
     });
     launch(c, "cols_inv_j", [&] { launch_cols(n, n, 0, +1, c->df_v, c->df_v, kp, n3, c->tw, s, c->cols_tile, c->cols_wide | kColsStream); });
     if (!c->df_pairs) {  // recompute the batch's filtered pairs
-      launch(c, "filter_i", [&] {
-        launch_filter_i(n, c->spec, c->ubuf, kk, n3, filter_weights(c), rb, c->tw, s, c->tile_filter,
-                        c->filter_pair);
-      });
+      enqueue_filter(c, rb, kk, false);
       launch(c, "cols_inv_j", [&] { launch_cols(n, n, 0, +1, c->ubuf, c->ubuf, kk, n3, c->tw, s, c->cols_tile, c->cols_wide | kColsStream); });
     }
     launch(c, "rows_seed", [&] {
@@ -1060,6 +1067,24 @@ bool noalloc_context(const sf21_hii_ctx* c) {
   return c->cfg.input_mode == SF21_INPUT_HALO && ng * ng * ng <= kNoAllocGrid;
 }
 
+// The FP32 weight table: the whole ladder where it takes at most 1/16 of the
+// memory that was free (free_b), else the radii that do, at most a batch and one
+// at least.  The last allocation of a context, so that it shrinks rather than
+// keep another one from fitting.  The plain path reads it in the inspection of
+// a filtered pair only: one radius.
+int make_w_table(sf21_hii_ctx* c, size_t free_b) {
+  const size_t one = (size_t)wtab_radius(c->n), nr = c->radii.size();
+  const size_t fit = free_b / 16 / (sizeof(float) * one);
+  const int batch = c->generic ? c->Kg : c->K;
+  c->Kw = c->cfg.path == SF21_PATH_PLAIN ? 1
+          : fit >= nr                    ? (int)nr
+                                         : std::max(1, (int)std::min(fit, (size_t)batch));
+  int rc;
+  while ((rc = dev_alloc(&c->wtab, one * c->Kw)) && c->Kw > 1) c->Kw = (c->Kw + 1) / 2;
+  if (!rc && c->Kw == (int)nr) launch_w_table(c->n, (int)nr, c->d_kappa, c->wtab, c->stream);
+  return rc;
+}
+
 // Deposit-only context: the stream and the parameters the deposit entry
 // points read; halo grid and sums are allocated on first use.
 int create_deposit(const sf21_hii_config* cfg, sf21_hii_ctx** out) {
@@ -1236,14 +1261,14 @@ int sf21_hii_create(const sf21_hii_config* cfg, sf21_hii_ctx** out) {
     c->rows_wide = tc.rw && wide_ok(c->n);
     c->filter_pair = tc.fp && tc.tile >= 8 && c->filter_w;
   }
+  size_t free_b = 0, total_b = 0;
+  if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = 0;
+  (void)hipGetLastError();
   if (cfg->path == SF21_PATH_FUSED && !c->generic && cfg->radius_batch <= 0 && !tuned) {
     // automatic batch: the whole ladder (the spectrum is read and transformed
     // along i once per batch: at 512^3 and 47 radii 11.2 ms of filter passes
     // per slice against 13.1 ms in batches of 16) while its pairs take at most
     // a third of the free memory, else halved down to 16
-    size_t free_b = 0, total_b = 0;
-    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = 0;
-    (void)hipGetLastError();
     c->K = (int)c->radii.size();
     while (c->K > 16 && sizeof(float2) * (size_t)c->n3 * c->K > free_b / 3) c->K = (c->K + 1) / 2;
     if (c->K < 16) c->K = 16;
@@ -1295,26 +1320,11 @@ int sf21_hii_create(const sf21_hii_config* cfg, sf21_hii_ctx** out) {
       rc = SF21_ERR_HIP;
       goto fail;
     }
-    if (c->filter_w && cfg->path == SF21_PATH_FUSED) {
-      // the FP32 weight table, if it takes at most 1/16 of the free memory
-      // (otherwise the filter pass evaluates the weights; generic sides fill a
-      // table of one batch, at most 16 GiB of pairs, before each batch)
-      const size_t nr = c->radii.size(), one = (size_t)wtab_radius(c->n);
-      size_t free_b = 0, total_b = 0;
-      if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = 0;
-      if (sizeof(float) * one * nr <= free_b / 16 && dev_alloc(&c->wtab, one * nr) == SF21_OK) {
-        c->wtab_all = true;
-        launch_w_table(c->n, (int)nr, c->d_kappa, c->wtab, c->stream);
-      }
-      if (c->generic) {
-        c->Kg = (int)nr;
-        const size_t pair = sizeof(float2) * (size_t)c->n3;
-        while (c->Kg > 1 && (pair * c->Kg > ((size_t)16 << 30) || pair * c->Kg > free_b / 3))
-          c->Kg = (c->Kg + 1) / 2;
-        if (!c->wtab_all)
-          while ((rc = dev_alloc(&c->wtab, one * c->Kg)) && c->Kg > 1) c->Kg = (c->Kg + 1) / 2;
-        if (rc) goto fail;
-      }
+    if (c->generic) {
+      c->Kg = (int)c->radii.size();
+      const size_t pair = sizeof(float2) * (size_t)c->n3;
+      while (c->Kg > 1 && (pair * c->Kg > ((size_t)16 << 30) || pair * c->Kg > free_b / 3))
+        c->Kg = (c->Kg + 1) / 2;
     }
     if ((rc = dev_alloc(&c->d_d2, c->d2.size()))) goto fail;
     if (hipMemcpy(c->d_d2, c->d2.data(), sizeof(int) * c->d2.size(), hipMemcpyHostToDevice) !=
@@ -1367,6 +1377,7 @@ int sf21_hii_create(const sf21_hii_config* cfg, sf21_hii_ctx** out) {
       goto fail;
   }
   if (noalloc_context(c) && (rc = ensure_halo_acc(c))) goto fail;
+  if (c->filter_w && (rc = make_w_table(c, free_b))) goto fail;
   // the tables are complete before any other stream can use them
   if (hipStreamSynchronize(c->stream) != hipSuccess || (rc = check_hip())) {
     if (!rc) rc = SF21_ERR_HIP;

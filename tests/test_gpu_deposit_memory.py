@@ -37,6 +37,8 @@ def test_sums_that_do_not_fit(torch_cuda):
     assert torch.equal(out[: 4 * n * n], first)
     for c in contexts:
         c.close()
+    del out
+    torch.cuda.empty_cache()
 
 
 def test_one_cell_blocks_take_no_sums(torch_cuda):
