@@ -78,8 +78,9 @@ typedef struct sf21_hii_config {
   int radius_batch;      /* radii per fused filter pass, 0 = automatic (the whole ladder
                             while its K n^3 complex buffer takes at most a third of the
                             free device memory, else fewer, 16 at least if they fit);
-                            sides without a register plan batch by themselves (at most
-                            16 GiB and a third of the free memory) and report 1 */
+                            sides without a register plan take at most 16 GiB and a
+                            third of the free memory, and no more radii than given
+                            here, for pairs and weights alike; they report 1 */
   int device;            /* HIP device ordinal */
   int filter_tile;       /* columns per block of the fused filter pass: 4, 8, 16 or 0 (auto) */
   int filter_w;          /* top-hat weights W(|k| R): 0 = automatic (FP32),

@@ -1069,15 +1069,19 @@ bool noalloc_context(const sf21_hii_ctx* c) {
 
 // The FP32 weight table: the whole ladder where it takes at most 1/16 of the
 // memory that was free (free_b), else the radii that do, at most a batch and one
-// at least.  The last allocation of a context, so that it shrinks rather than
+// at least.  With a radius batch given on a side without a register plan, whose
+// passes always need a table, the caller bounds it too: no more than the batch's
+// pairs take (8 times a radius' weights).  The last allocation of a context, so that it shrinks rather than
 // keep another one from fitting.  The plain path reads it in the inspection of
 // a filtered pair only: one radius.
 int make_w_table(sf21_hii_ctx* c, size_t free_b) {
   const size_t one = (size_t)wtab_radius(c->n), nr = c->radii.size();
   const size_t fit = free_b / 16 / (sizeof(float) * one);
   const int batch = c->generic ? c->Kg : c->K;
+  const bool bounded = c->generic && c->cfg.radius_batch > 0;
+  const bool whole = fit >= nr && (!bounded || nr <= (size_t)8 * batch);
   c->Kw = c->cfg.path == SF21_PATH_PLAIN ? 1
-          : fit >= nr                    ? (int)nr
+          : whole                        ? (int)nr
                                          : std::max(1, (int)std::min(fit, (size_t)batch));
   int rc;
   while ((rc = dev_alloc(&c->wtab, one * c->Kw)) && c->Kw > 1) c->Kw = (c->Kw + 1) / 2;
@@ -1325,6 +1329,7 @@ int sf21_hii_create(const sf21_hii_config* cfg, sf21_hii_ctx** out) {
       const size_t pair = sizeof(float2) * (size_t)c->n3;
       while (c->Kg > 1 && (pair * c->Kg > ((size_t)16 << 30) || pair * c->Kg > free_b / 3))
         c->Kg = (c->Kg + 1) / 2;
+      if (cfg->radius_batch > 0) c->Kg = std::min(c->Kg, cfg->radius_batch);
     }
     if ((rc = dev_alloc(&c->d_d2, c->d2.size()))) goto fail;
     if (hipMemcpy(c->d_d2, c->d2.data(), sizeof(int) * c->d2.size(), hipMemcpyHostToDevice) !=

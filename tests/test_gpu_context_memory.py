@@ -45,3 +45,28 @@ def test_plain_path_filtered_pair(torch_cuda):
         pairs.append(ctx.filtered(a, b, radius_index=3))
         ctx.close()
     assert torch.equal(*pairs)
+
+
+@pytest.mark.parametrize("K", [1, 3, 1000])
+def test_radius_batch_bounds_a_line_side(torch_cuda, K):
+    """On a side without a register plan radius_batch bounds the pairs and the
+    weights; the slice stays the same."""
+    torch = torch_cuda
+    n, nr = 240, 40
+    g = torch.Generator(device="cuda")
+    g.manual_seed(K)
+    a = torch.exp(0.8 * torch.randn(n ** 3, generator=g, device="cuda"))
+    b = torch.exp(1.2 * torch.randn(n ** 3, generator=g, device="cuda") - 0.3)
+    b *= torch.rand(n ** 3, generator=g, device="cuda") < 0.3
+    got = []
+    for k in (0, K):
+        ctx = sf.HiiContext(n, 1.5 * n, ladder(n, nr), sf.INPUT_DIRECT, sf.PATH_FUSED, radius_batch=k)
+        x, mean = ctx.run_slice(a, b)
+        got.append((x, mean, np.asarray(ctx.weight_map()).copy()))
+        ctx.close()
+    assert torch.equal(got[0][0], got[1][0]) and got[0][1] == got[1][1]
+    assert np.array_equal(got[0][2], got[1][2]) and 0 < (got[0][2] >= 0).sum() < n ** 3
+    # pairs and at most as much for the weights, the spectrum, two integer maps
+    held(torch, n, ladder(n, 2))
+    bound = (2 * min(K, nr) + 2) * 8 * n ** 3 + SLACK
+    assert held(torch, n, ladder(n, nr), radius_batch=K) <= bound
