@@ -77,7 +77,9 @@ typedef struct sf21_hii_config {
   double fesc;           /* escape fraction, SFR mode (get_HIIbubbles.c:273) */
   int radius_batch;      /* radii per fused filter pass, 0 = automatic (the whole ladder
                             while its K n^3 complex buffer takes at most a third of the
-                            free device memory, else fewer, 16 at least if they fit);
+                            free device memory, else fewer, 16 at least if they fit;
+                            down to 16 later where the differentiable mode's stored
+                            fields need the room);
                             sides without a register plan take at most 16 GiB and a
                             third of the free memory, and no more radii than given
                             here, for pairs and weights alike; they report 1 */

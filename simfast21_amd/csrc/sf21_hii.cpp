@@ -870,6 +870,48 @@ void enqueue_diff_backward_generic(sf21_hii_ctx* c, const float* g, const float*
   });
 }
 
+// Called whenever a context's buffers, stream or kernel choices change: its
+// own graphs go, and the new generation keeps multi-box graphs cached on
+// other contexts from replaying the old state.
+void drop_graphs(sf21_hii_ctx* c) {
+  for (auto& g : c->graphs)
+    if (g.exec) (void)hipGraphExecDestroy(g.exec);
+  c->graphs.clear();
+  c->gen++;
+}
+
+// Change the radius batch: the K n^3 pair buffer (and the differentiable
+// mode's (K+1)/2 n^3 ball-pair buffer) are reallocated.
+int set_radius_batch(sf21_hii_ctx* c, int K) {
+  if (K > (int)c->radii.size()) K = (int)c->radii.size();
+  if (K < 1) return SF21_ERR_ARG;
+  if (K == c->K && K == c->Kd) return SF21_OK;
+  if (hipStreamSynchronize(c->stream) != hipSuccess) return SF21_ERR_HIP;
+  drop_graphs(c);
+  dev_free(c->ubuf);
+  int rc = dev_alloc(&c->ubuf, (size_t)c->n3 * K);
+  if (rc) {
+    // keep the context usable with its previous batch
+    if (dev_alloc(&c->ubuf, (size_t)c->n3 * c->K)) return SF21_ERR_ALLOC;
+    return rc;
+  }
+  c->K = c->Kd = K;
+  if (c->df_v) {
+    dev_free(c->df_v);
+    if ((rc = dev_alloc(&c->df_v, (size_t)(c->Kd + 1) / 2 * c->n3))) {
+      c->df_ready = false;
+      return rc;
+    }
+  }
+  return SF21_OK;
+}
+
+// Gives back what the automatic batch holds beyond the radii that the
+// differentiable backward takes at a time; false if there is nothing to give.
+bool shrink_batch(sf21_hii_ctx* c) {
+  return !c->generic && c->Kd < c->K && set_radius_batch(c, c->Kd) == SF21_OK;
+}
+
 int diff_check(sf21_hii_ctx* c, const float* g, const float* emis, int nbins) {
   if (!c || !g || !emis || nbins < 1 || nbins > 64) return SF21_ERR_ARG;
   if (c->cfg.input_mode != SF21_INPUT_DIRECT || c->cfg.path != SF21_PATH_FUSED) return SF21_ERR_ARG;
@@ -881,10 +923,15 @@ int diff_check(sf21_hii_ctx* c, const float* g, const float* emis, int nbins) {
   if ((rc = ensure_diff(c))) return rc;
   if (c->df_store == 2 && !c->df_pairs && !c->generic) {
     // automatic field storage: keep the pairs when they take at most half
-    // of the free device memory
+    // of the free device memory, after the automatic batch has given back its
+    // share if it takes that
     size_t free_b = 0, total_b = 0;
-    const size_t need = sizeof(float2) * (size_t)c->n3 * c->radii.size();
-    if (hipMemGetInfo(&free_b, &total_b) == hipSuccess && need <= free_b / 2 &&
+    const size_t pair = sizeof(float2) * (size_t)c->n3, need = pair * c->radii.size();
+    if (hipMemGetInfo(&free_b, &total_b) == hipSuccess && need > free_b / 2 &&
+        need <= (free_b + pair * (c->K - c->Kd)) / 2 && shrink_batch(c) &&
+        hipMemGetInfo(&free_b, &total_b) != hipSuccess)
+      free_b = 0;
+    if (need <= free_b / 2 &&
         dev_alloc(&c->df_pairs, (size_t)c->n3 * c->radii.size()) != SF21_OK)
       c->df_pairs = nullptr;
     (void)hipGetLastError();
@@ -985,42 +1032,6 @@ void tune_store_gen(const char* path, const std::string& key, int gx, double ms)
   if (!f) return;
   std::fprintf(f, "%s | gx=%d | %.3f ms\n", key.c_str(), gx, ms);
   std::fclose(f);
-}
-
-// Called whenever a context's buffers, stream or kernel choices change: its
-// own graphs go, and the new generation keeps multi-box graphs cached on
-// other contexts from replaying the old state.
-void drop_graphs(sf21_hii_ctx* c) {
-  for (auto& g : c->graphs)
-    if (g.exec) (void)hipGraphExecDestroy(g.exec);
-  c->graphs.clear();
-  c->gen++;
-}
-
-// Change the radius batch: the K n^3 pair buffer (and the differentiable
-// mode's (K+1)/2 n^3 ball-pair buffer) are reallocated.
-int set_radius_batch(sf21_hii_ctx* c, int K) {
-  if (K > (int)c->radii.size()) K = (int)c->radii.size();
-  if (K < 1) return SF21_ERR_ARG;
-  if (K == c->K && K == c->Kd) return SF21_OK;
-  if (hipStreamSynchronize(c->stream) != hipSuccess) return SF21_ERR_HIP;
-  drop_graphs(c);
-  dev_free(c->ubuf);
-  int rc = dev_alloc(&c->ubuf, (size_t)c->n3 * K);
-  if (rc) {
-    // keep the context usable with its previous batch
-    if (dev_alloc(&c->ubuf, (size_t)c->n3 * c->K)) return SF21_ERR_ALLOC;
-    return rc;
-  }
-  c->K = c->Kd = K;
-  if (c->df_v) {
-    dev_free(c->df_v);
-    if ((rc = dev_alloc(&c->df_v, (size_t)(c->Kd + 1) / 2 * c->n3))) {
-      c->df_ready = false;
-      return rc;
-    }
-  }
-  return SF21_OK;
 }
 
 bool wide_ok(int n) { return n == 128 || n == 256 || n == 512; }
@@ -2214,7 +2225,10 @@ int sf21_hii_diff_store_fields(sf21_hii_ctx* c, int mode) {
     return SF21_OK;
   }
   if (c->df_pairs || mode == 2) return SF21_OK;  // automatic: decided at the next backward
-  return dev_alloc(&c->df_pairs, (size_t)c->n3 * c->radii.size());
+  const size_t count = (size_t)c->n3 * c->radii.size();
+  int rc = dev_alloc(&c->df_pairs, count);
+  if (rc && shrink_batch(c)) rc = dev_alloc(&c->df_pairs, count);
+  return rc;
 }
 
 int sf21_hii_diff_last_kept(const sf21_hii_ctx* c) {

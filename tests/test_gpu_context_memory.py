@@ -70,3 +70,33 @@ def test_radius_batch_bounds_a_line_side(torch_cuda, K):
     held(torch, n, ladder(n, 2))
     bound = (2 * min(K, nr) + 2) * 8 * n ** 3 + SLACK
     assert held(torch, n, ladder(n, nr), radius_batch=K) <= bound
+
+
+def test_automatic_batch_makes_room_for_stored_fields(torch_cuda):
+    """The finder's automatic batch gives its memory back where the
+    differentiable mode's stored fields would otherwise not fit."""
+    torch = torch_cuda
+    torch.cuda.empty_cache()
+    n = 256
+    pair, total = 8 * n ** 3, torch.cuda.mem_get_info()[1]
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(3)
+    g = 0.5 * torch.randn(n ** 3, generator=gen, device="cuda")
+    emis = torch.rand(n ** 3, generator=gen, device="cuda")
+    # automatic storage: fields of 0.36 of the memory fit half of what 16 pairs
+    # leave free, and not half of what a third of the memory leaves
+    nr = int(0.36 * total / pair)
+    ctx = sf.HiiContext(n, 1.5 * n, ladder(n, nr), sf.INPUT_DIRECT, sf.PATH_FUSED)
+    assert ctx.radius_batch > 100
+    ctx.diff_backward(g, emis, 1.5, 0.02, 1.0, None)
+    ctx.profile(True)
+    ctx.diff_backward(g, emis, 1.5, 0.02, 1.0, None)
+    # one sweep of filter passes: the second reads the stored fields
+    assert ctx.kernel_stats()["filter_i"][0] == (nr + 15) // 16
+    ctx.close()
+    # storage asked for: 0.8 of the memory
+    ctx = sf.HiiContext(n, 1.5 * n, ladder(n, int(0.8 * total / pair)), sf.INPUT_DIRECT, sf.PATH_FUSED)
+    assert ctx.radius_batch > 100
+    ctx.diff_store_fields(1)
+    assert ctx.radius_batch == 16
+    ctx.close()
