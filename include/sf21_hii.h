@@ -275,13 +275,14 @@ int sf21_hii_filtered_dev(sf21_hii_ctx *ctx, const float *a, const float *b, con
 
 /* Autotuner (fused path; no counterpart in the reference, whose FFTW plans
  * are tuned by FFTW_MEASURE at get_HIIbubbles.c:110-183).  Times the slice
- * (a, b, c, z; device pointers) by a coordinate search over launch shapes
- * and stage orders: radius batch 16, 8, 12, 24, 32 or the whole ladder
- * (capped by the ladder; skipped when it does not fit), filter tile 16/8, filter blocks over single
- * i-lines or mirror pairs (kj, n - kj) sharing W, the per-radius column
- * passes (8 values per thread with 8 or 16 columns per block, or 16 values
- * per thread with 16 or 32 columns, the latter for n = 128, 256, 512; with
- * 16 or 32 columns also as blocks that walk 8 tiles and prefetch the next)
+ * (a, b, c, z; device pointers) by a coordinate search from the choices in
+ * force over launch shapes and stage orders: radius batch 8, 12, 16, 24, 32
+ * or the whole ladder (capped by the ladder; skipped when it does not fit),
+ * filter tile 8/16, filter blocks in order or mirror lines (kj, n - kj),
+ * which read the same weights, together, the per-radius column passes (8
+ * values per thread with 8 or 16 columns per block, or 16 values per thread
+ * with 16 or 32 columns, the latter for n = 128, 256, 512; with 16 or 32
+ * columns also as blocks that walk 8 tiles and prefetch the next)
  * and the centre-test pass (8 or 16 values per thread).  The top-hat weight
  * mode (filter_w) is never searched: it stays what the configuration says.
  * Keeps the fastest in the context and appends it to the cache file
@@ -299,8 +300,8 @@ int sf21_hii_autotune(sf21_hii_ctx *ctx, const float *a, const float *b, const f
 /* Current choices: filter tile, radius batch, top-hat weights (1 FP32, 2
  * from FP64), column-pass tile, column-pass variant (bit 0: 16 values
  * per thread, bit 1: prefetching blocks), 16 values per thread in the
- * centre-test pass (0/1), filter blocks over mirror pairs of i-lines that
- * share the weights (0/1); any pointer may be NULL. */
+ * centre-test pass (0/1), filter blocks of mirror i-lines, which read the
+ * same weights, together (0/1); any pointer may be NULL. */
 int sf21_hii_tuning(const sf21_hii_ctx *ctx, int *filter_tile, int *radius_batch, int *filter_w,
                     int *cols_tile, int *cols_wide, int *rows_wide, int *filter_pair);
 

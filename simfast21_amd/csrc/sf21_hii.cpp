@@ -14,6 +14,7 @@
 #include "../../include/sf21_hii.h"
 #include "host_params.h"
 #include "kernels.h"
+#include "tune_search.h"
 
 using namespace sf21;
 
@@ -888,12 +889,14 @@ int set_radius_batch(sf21_hii_ctx* c, int K) {
   if (K == c->K && K == c->Kd) return SF21_OK;
   if (hipStreamSynchronize(c->stream) != hipSuccess) return SF21_ERR_HIP;
   drop_graphs(c);
-  dev_free(c->ubuf);
-  int rc = dev_alloc(&c->ubuf, (size_t)c->n3 * K);
-  if (rc) {
-    // keep the context usable with its previous batch
-    if (dev_alloc(&c->ubuf, (size_t)c->n3 * c->K)) return SF21_ERR_ALLOC;
-    return rc;
+  int rc;
+  if (K != c->K) {
+    dev_free(c->ubuf);
+    if ((rc = dev_alloc(&c->ubuf, (size_t)c->n3 * K))) {
+      // keep the context usable with its previous batch
+      if (dev_alloc(&c->ubuf, (size_t)c->n3 * c->K)) return SF21_ERR_ALLOC;
+      return rc;
+    }
   }
   c->K = c->Kd = K;
   if (c->df_v) {
@@ -939,14 +942,7 @@ int diff_check(sf21_hii_ctx* c, const float* g, const float* emis, int nbins) {
   return SF21_OK;
 }
 
-// ---- autotuner: choices of the fused path, persisted per (arch, n, radii) ----
-// Only choices that change launch shapes and stage order are searched; the
-// top-hat weight mode (in-kernel FP32 or the FP64 table) changes values and
-// stays an explicit configuration setting.
-struct TuneChoice {
-  int tile = 16, K = 16, ct = 16, cw = 0, rw = 0, fp = 0;
-};
-
+// ---- autotuner: choices of the fused path (tune_search.h), persisted per (arch, n, radii) ----
 std::string tune_key(const sf21_hii_ctx* c) {
   hipDeviceProp_t prop;
   std::string arch = "unknown";
@@ -1032,18 +1028,6 @@ void tune_store_gen(const char* path, const std::string& key, int gx, double ms)
   if (!f) return;
   std::fprintf(f, "%s | gx=%d | %.3f ms\n", key.c_str(), gx, ms);
   std::fclose(f);
-}
-
-bool wide_ok(int n) { return n == 128 || n == 256 || n == 512; }
-
-
-// Column-pass variant that exists for this size and tile: 16 values per
-// thread only for wide_ok sizes (tile 16 or 32), prefetching blocks only
-// with tile 16 (8 values) or tile 32 (16 values).
-int cols_variant(int n, int tile, int cw) {
-  const bool wide = (cw & 1) && wide_ok(n) && (tile == 16 || tile == 32);
-  const bool pipe = (cw & 2) && (tile == 16 || (wide && tile == 32));
-  return (wide ? 1 : 0) | (pipe ? 2 : 0);
 }
 
 void apply_choice(sf21_hii_ctx* c, const TuneChoice& t) {
@@ -1760,67 +1744,14 @@ int sf21_hii_autotune(sf21_hii_ctx* c, const float* a, const float* b, const flo
     *ms_out = ms / 2;
     return 0;
   };
-  // coordinate search from the defaults: each dimension in turn, the others
-  // held at the best so far
-  const int nr = (int)c->radii.size();
-  TuneChoice best;
-  best.K = std::min(16, nr);
-  double best_t = 1e300;
-  {
-    double ms;
-    int r0 = timed(best, &ms);
-    if (r0 < 0) rc = SF21_ERR_HIP;
-    else if (r0 == 0) best_t = ms;
-  }
-  auto consider = [&](TuneChoice t) {
-    if (rc) return;
-    double ms;
-    int r1 = timed(t, &ms);
-    if (r1 < 0) rc = SF21_ERR_HIP;
-    else if (r1 == 0 && ms < best_t) {
-      best_t = ms;
-      best = t;
-    }
-  };
-  // larger batches read the spectrum fewer times per slice; candidates that
-  // do not fit in device memory are skipped
-  for (int K : {8, 12, 24, 32, nr}) {
-    TuneChoice t = best;
-    t.K = std::min(K, nr);
-    if (t.K != best.K) consider(t);
-  }
-  {
-    TuneChoice t = best;
-    t.tile = 8;
-    consider(t);
-  }
-  {
-    TuneChoice t = best;
-    t.fp = 1 - t.fp;
-    consider(t);
-  }
-  if (!c->plane) {  // plane sides have neither a j pass nor a p pass
-    const TuneChoice base = best;
-    const int cols_opts[7][2] = {{8, 0}, {16, 0}, {16, 2}, {16, 1}, {16, 3}, {32, 1}, {32, 3}};
-    for (auto& o : cols_opts) {
-      if ((o[1] & 1) && !wide_ok(c->n)) continue;
-      TuneChoice t = base;
-      t.ct = o[0];
-      t.cw = o[1];
-      if (t.ct != base.ct || t.cw != base.cw) consider(t);
-    }
-  }
-  if (!c->plane && wide_ok(c->n)) {
-    TuneChoice t = best;
-    t.rw = 1;
-    consider(t);
-  }
+  TuneChoice best{c->tile_filter, c->K, c->cols_tile, c->cols_wide, c->rows_wide ? 1 : 0, c->filter_pair};
+  double best_t = 0.0;
+  const int found = tune_search(c->n, (int)c->radii.size(), c->plane, timed, &best, &best_t);
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   dev_free(xout);
   c->prof = prof;
-  if (rc) return rc;
-  if (best_t >= 1e300) return SF21_ERR_ALLOC;
+  if (found) return found < 0 ? SF21_ERR_HIP : SF21_ERR_ALLOC;
   if ((rc = set_radius_batch(c, best.K))) return rc;
   apply_choice(c, best);
   tune_store(tune_path(cache_path), tune_key(c), best, best_t);
