@@ -1053,7 +1053,9 @@ static int radius_groups(long waves, int nrad) {
 
 void launch_w_table(int n, int nr, const float2* kappa, float* wt, hipStream_t s) {
   const int g = n % 16 == 0 ? 16 : 8;
-  hipLaunchKernelGGL(k_w_table, dim3(n / g, n / 2 + 1, nr), dim3(256), 0, s, n, kappa, wt);
+  for (int r = 0; r < nr; r += 32768)  // a grid holds at most 65535 along z
+    hipLaunchKernelGGL(k_w_table, dim3(n / g, n / 2 + 1, nr - r < 32768 ? nr - r : 32768), dim3(256),
+                       0, s, n, kappa + r, wt + r * wtab_radius(n));
 }
 
 void launch_filter_i(int n, const float2* spec, float2* u, int nrad, long ustride,

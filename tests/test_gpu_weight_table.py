@@ -33,6 +33,17 @@ def test_long_ladder_equals_its_parts(torch_cuda, n):
     assert np.array_equal(w, parts)
 
 
+@pytest.mark.parametrize("n", [16, 32])
+def test_more_radii_than_a_grid_has_planes(torch_cuda, n):
+    """65600 radii, five different ones: the map of those five."""
+    side = 1.5 * n
+    radii = np.geomspace(0.25 * side, 2.0, 5)
+    a, b = boxes(torch_cuda, n, 80 + n)
+    w = centre_map(n, side, list(radii), a, b)
+    assert 0 < (w >= 0).sum() < n ** 3
+    assert np.array_equal(centre_map(n, side, list(np.repeat(radii, 13120)), a, b), w)
+
+
 def test_same_bits_with_little_free_memory(torch_cuda):
     torch = torch_cuda
     n, side, room = 512, 768.0, 85 << 30
