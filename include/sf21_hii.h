@@ -146,8 +146,10 @@ int sf21_hii_halo_emissivity_dev(sf21_hii_ctx *ctx, const float *halos, long n_h
  * hipMalloc).  Same arguments and result (the same kernels); the n^3 FP64
  * sums live in a buffer that the context allocates when it is created
  * (sf21_hii_create fails if it cannot; for input_mode SF21_INPUT_HALO and
- * N_halo <= 256, larger grids -> SF21_ERR_ARG).  Enqueued on the context's stream without host
- * synchronisation. */
+ * N_halo <= 256, larger grids -> SF21_ERR_ARG).  Enqueued on the context's
+ * stream without host synchronisation.  Calls on one context share that
+ * buffer: two that overlap in time (graphs captured from one context and
+ * launched on different streams) race; calls on different contexts do not. */
 int sf21_hii_halo_emissivity_noalloc(sf21_hii_ctx *ctx, const float *halos, long n_halos,
                                      double z, float *ion_out);
 int sf21_hii_run_slice_halo(sf21_hii_ctx *ctx, const float *delta, const float *halos,
