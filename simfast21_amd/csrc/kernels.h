@@ -92,9 +92,7 @@ struct FilterW {
 constexpr long wtab_radius(int n) { return (long)(n / 2 + 1) * (n / 2 + 1) * n; }
 void launch_w_table(int n, int nr, const float2* kappa, float* wt, hipStream_t s);
 // mirror: the block order that runs the i-lines kj and n - kj, which share their
-// weights, together on one XCD;
-// t16: u in the 16-column tile layout of launch_cols (the p pass then reads
-// it with t16 as well)
+// weights, together on one XCD; t16: u in the 16-column tile layout of launch_cols
 void launch_filter_i(int n, const float2* spec, float2* u, int nrad, long ustride,
                      const FilterW& w, const float2* tw, hipStream_t s, int tile, bool mirror,
                      bool t16);
@@ -105,10 +103,10 @@ bool plane_prepare(int n);
 void launch_plane_crit(int n, const float2* u, int nrad, long ustride, const int* d2max,
                        const float* bal, int* wmap, float2* dbg, float2* keep, const float2* tw,
                        hipStream_t s);
+// u in the tile layout; wide: 16 values per thread (256, 512)
 void launch_inv_rows_crit(int n, const float2* v, int nrad, long vstride, const int* d2max,
                           const float* bal, int* wmap, float2* dbg, hipStream_t s,
-                          const float2* tw, bool wide = false,
-                          float2* keep = nullptr, bool t16 = false);
+                          const float2* tw, bool wide, float2* keep);
 void launch_fill_i32(int* p, int value, long count, hipStream_t s);
 // cells per lane of the dilation line passes for box side n (0: n not usable)
 int dt_q(int n);

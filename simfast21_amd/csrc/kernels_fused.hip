@@ -423,8 +423,8 @@ __global__ __launch_bounds__(TILE*(L / Plan<L>::E)) void k_filter_lut(
 }
 
 // ------------------------------------------------------------------------
-// Per radius batch: inverse along p -> (N^3 rec_R, s N^3 ion_R) for each of
-// the nrad radii, centre test, and for every cell the largest ball bound
+// Per radius batch, buffer in the tile layout: inverse along p -> (N^3 rec_R, s
+// N^3 ion_R) for each of the nrad radii, centre test, and for every cell the largest ball bound
 // among the batch's radii at which it is a centre.  Batches are issued in
 // ascending radius, so a batch's bounds exceed every earlier batch's and a
 // plain store (only where some centre was found) leaves in wmap the bound of
@@ -444,7 +444,7 @@ __global__ __launch_bounds__(256) void k_inv_rows_crit(const float2* __restrict_
                                                        int* __restrict__ wmap,
                                                        float2* __restrict__ dbg,
                                                        float2* __restrict__ keep,
-                                                       const float2* __restrict__ tw, int t16) {
+                                                       const float2* __restrict__ tw) {
   constexpr int TPL = L / E, LPB = 256 / TPL;
   static_assert(L % LPB == 0 && TPL % 16 == 0, "the block's rows in one plane, whole tiles");
   __shared__ float lds[LPB * 2 * LdsLine<L>::kFloats];
@@ -457,21 +457,15 @@ __global__ __launch_bounds__(256) void k_inv_rows_crit(const float2* __restrict_
   const float sc = bal[0];
   // element p = t + TPL m of the row sits at voff plus a step in m of the plane:
   // a per-thread offset plus a uniform one (scalar address arithmetic).
-  const unsigned voff = t16 ? 16 * j + (unsigned)t16_tile<L>(0, t >> 4) + (t & 15) : j * L + t;
+  const unsigned voff = 16 * j + (unsigned)t16_tile<L>(0, t >> 4) + (t & 15);
   int wbest[E];
 #pragma unroll
   for (int m = 0; m < E; ++m) wbest[m] = -1;
   float2 nx[E];
   auto fetch = [&](int r) {
-    const float2* __restrict__ src =
-        vin + (long)r * vstride + (t16 ? t16_tile<L>(plane, 0) : (long)plane * (L * L));
-    if (t16) {
+    const float2* __restrict__ src = vin + (long)r * vstride + t16_tile<L>(plane, 0);
 #pragma unroll
-      for (int m = 0; m < E; ++m) nx[m] = ld_stream(uniform_ptr(src + m * TPL * L * L) + voff);
-    } else {
-#pragma unroll
-      for (int m = 0; m < E; ++m) nx[m] = ld_stream(uniform_ptr(src + TPL * m) + voff);
-    }
+    for (int m = 0; m < E; ++m) nx[m] = ld_stream(uniform_ptr(src + m * TPL * L * L) + voff);
   };
   TwRegs<L, E> wr;
   wr.load(t, tw);
@@ -1142,20 +1136,19 @@ void launch_plane_crit(int n, const float2* u, int nrad, long ustride, const int
 
 void launch_inv_rows_crit(int n, const float2* v, int nrad, long vstride, const int* d2max,
                           const float* bal, int* wmap, float2* dbg, hipStream_t s,
-                          const float2* tw, bool wide, float2* keep, bool t16) {
-  const int lay = t16 ? 1 : 0;
+                          const float2* tw, bool wide, float2* keep) {
 #define XW(L)                                                                             \
   if (n == L && wide) {                                                                   \
     constexpr int LPB = 256 / (L / 16);                                                   \
     hipLaunchKernelGGL((k_inv_rows_crit<L, 16>), dim3((L * L) / LPB), dim3(256), 0, s, v, nrad, \
-                       vstride, d2max, bal, wmap, dbg, keep, tw, lay);                          \
+                       vstride, d2max, bal, wmap, dbg, keep, tw);                               \
     return;                                                                               \
   }
 #define X(L)                                                                              \
   if (n == L) {                                                                           \
     constexpr int LPB = 256 / (L / Plan<L>::E);                                           \
     hipLaunchKernelGGL(k_inv_rows_crit<L>, dim3((L * L) / LPB), dim3(256), 0, s, v, nrad, vstride, \
-                       d2max, bal, wmap, dbg, keep, tw, lay);                                   \
+                       d2max, bal, wmap, dbg, keep, tw);                                        \
     return;                                                                               \
   }
   XW(256) XW(512)

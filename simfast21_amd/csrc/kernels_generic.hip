@@ -44,7 +44,7 @@ __device__ __forceinline__ void gen_twiddle(float2* a, int k, int tstep,
   }
 }
 
-// First stage (radix 8, NS = 1): inputs from HBM (times W(|k| R) in mode 1).
+// First stage (radix 8, NS = 1): inputs from HBM.
 // Output position o = 8 j + r is kept transposed, at slot r L/8 + j, so that
 // the stores of consecutive butterflies are consecutive (a stride-8 store
 // pattern conflicts in the LDS banks); the next stage reads position o at
@@ -53,24 +53,15 @@ __device__ __forceinline__ int gen_t1_slot(int o, int lr0) { return (o & 7) * lr
 
 // LC (and NSC): the side (and the stage span) as compile-time constants for
 // the specialised sides, 0 for the runtime plan.
-template <int R, int SIGN, int MODE, int LC>
+template <int R, int SIGN, int LC>
 __device__ __forceinline__ void gen_first(const GenPlan& P, int jj, float2* line,
-                                          const float2* src, unsigned base, unsigned stride,
-                                          int msq, float2 kappa) {
+                                          const float2* src, unsigned base, unsigned stride) {
   const int L = LC ? LC : P.L, Lr = L / R;
 #pragma unroll 2
   for (int j = jj; j < Lr; j += 32) {
     float2 a[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int e = j + r * Lr;
-      float2 v = src[base + (unsigned)e * stride];
-      if constexpr (MODE == 1) {
-        const float w = w_tophat_k(kappa, msq + fold_sq(e, L));
-        v = make_float2(v.x * w, v.y * w);
-      }
-      a[r] = v;
-    }
+    for (int r = 0; r < R; ++r) a[r] = src[base + (unsigned)(j + r * Lr) * stride];
     Dft<R, SIGN>::run(a);
 #pragma unroll
     for (int r = 0; r < R; ++r) line[r * Lr + j] = a[r];
@@ -83,8 +74,7 @@ __device__ __forceinline__ void gen_first(const GenPlan& P, int jj, float2* line
 // lines depends on |k|^2 = msq_l + fold(e)^2, so it is evaluated once per
 // (line, |fold(e)|) -- 8 (L/2 + 1) values instead of 8 L -- into a table in
 // the line buffers, which the stage's stores overwrite only after every
-// thread has multiplied its inputs.  The same function of the same |k|^2 as
-// the direct evaluation: identical values.  The first radix is 8, so a
+// thread has multiplied its inputs.  The first radix is 8, so a
 // thread holds at most (768/8 + 31)/32 = 3 butterflies.
 template <int SIGN, int LC>
 __device__ __forceinline__ void gen_first_wtab(const GenPlan& P, float2* gsm, float2* line,
@@ -212,7 +202,6 @@ __global__ __launch_bounds__(256, 4) void k_gen_pass(const float2* src, float2* 
   const int l = ROWS ? (int)(threadIdx.x >> 5) : (int)(threadIdx.x & 7);
   const int jj = ROWS ? (int)(threadIdx.x & 31) : (int)(threadIdx.x >> 3);
   unsigned base, stride;
-  int msq = 0;  // |k|^2 of the two coordinates fixed along the line
   if (ROWS) {
     const unsigned row = blk * kGenLines + l;
     base = row * L;
@@ -223,7 +212,6 @@ __global__ __launch_bounds__(256, 4) void k_gen_pass(const float2* src, float2* 
     const unsigned p = (blk % ntile) * kGenLines + l;
     base = axis == 1 ? outer * L2 + p : outer * L + p;
     stride = axis == 1 ? L : L2;
-    if (MODE == 1) msq = fold_sq((int)outer, (int)L) + fold_sq((int)p, (int)L);
   }
   float2* line = gsm + l * (LC == 600 ? 616 : plan.lp);
   // the first radix is 8 on every generic side (multiples of 8)
@@ -234,7 +222,7 @@ __global__ __launch_bounds__(256, 4) void k_gen_pass(const float2* src, float2* 
                              fold_sq((int)(blk / ntile), (int)L),
                              (int)((blk % ntile) * kGenLines), kappa);
   } else {
-    gen_first<8, SIGN, MODE, LC>(plan, jj, line, src, base, stride, msq, kappa);
+    gen_first<8, SIGN, LC>(plan, jj, line, src, base, stride);
   }
   if constexpr (LC == 600) {
     gen_mid<3, SIGN, true, 600, 8>(plan, 1, jj, line, tw);

@@ -409,7 +409,7 @@ void enqueue_fused(sf21_hii_ctx* c, const float* a, const float* b, const float*
     });
     launch(c, "inv_rows_crit", [&] {
       launch_inv_rows_crit(n, c->ubuf, kk, n3, c->d_d2 + rb, c->bal, c->wmap, dbg, s, c->tw, c->rows_wide,
-                           keep ? keep + (long)rb * n3 : nullptr, true);
+                           keep ? keep + (long)rb * n3 : nullptr);
     });
   }
   if (only_radius >= 0) return;
