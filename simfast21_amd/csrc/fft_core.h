@@ -20,10 +20,14 @@
 
 namespace sf21 {
 
-// The products and sums of the transforms are spelled out as roundings and
-// fused multiply-adds instead of being left to the compiler's contraction,
-// which chooses by basic block: the centre test is discontinuous, so the same
-// line has to come out bit for bit in every kernel that carries it.
+// The centre test is discontinuous, so a line has to come out bit for bit in every
+// kernel of the finder that carries it, and the compiler's contraction of products
+// and sums chooses by basic block.  The twiddle products of the radius loops
+// (cmul_fixed) and Dft<8> therefore spell out which products are rounded and which
+// fused, as does the centre-test passes' last stage (ROUND).  Left to the compiler:
+// cmul in stages() (forward transforms, generic line passes, the differentiable
+// mode), Dft<5>, the first sum of Dft<3>, and the product by W in the filter pass of
+// the register-plan sides, of which there is one kernel per weight mode.
 __device__ __forceinline__ float2 cmul(float2 a, float2 b) {
   return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
@@ -32,8 +36,10 @@ __device__ __forceinline__ float mul_rounded(float a, float b) {
 #pragma clang fp contract(off)
   return a * b;
 }
-// cmul with its roundings spelled out: the form the compiler gives cmul in
-// every radix-8 plan (each component's a*b.y product rounded, the other fused)
+// cmul with its roundings spelled out (each component's a*b.y product rounded, the
+// other fused): the form that this compiler gives cmul in the radix-8 plans, so
+// that stages() and loop_stages() agree there; the tests of the launch choices and
+// of the radius batches compare kernels of both
 __device__ __forceinline__ float2 cmul_fixed(float2 a, float2 b) {
   return make_float2(fmaf(a.x, b.x, -mul_rounded(a.y, b.y)), fmaf(a.y, b.x, mul_rounded(a.x, b.y)));
 }
@@ -157,7 +163,7 @@ __device__ __forceinline__ void st_stream(float2* p, float2 a) {
 
 // Compiler-level fence for the LDS exchanges.  __syncthreads() orders the
 // hardware, but the compiler was observed to sink a stage's LDS reads past
-// the following barrier into a later basic block (k_filter_i: the forward
+// the following barrier into a later basic block (the filter pass: the forward
 // transform's last reads landed after the barrier, racing with the inverse
 // transform's first LDS writes of another wave).  An empty asm with a memory
 // clobber pins every LDS access of an exchange on its side of the barrier.

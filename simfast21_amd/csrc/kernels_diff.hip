@@ -522,7 +522,7 @@ __global__ __launch_bounds__(TILE*(L / Plan<L>::E)) void k_filter_acc_i(
 #pragma unroll
     for (int m = 0; m < E; ++m) v[m] = src[(tl + TPL * m) * (L * L)];
     line_fft<L, -1>(v, sre, sim, tl, tw);
-    // the same W_R as the forward pass (k_filter_i): table or FP32 evaluation
+    // the same W_R as the forward's weights: from FP64 or evaluated in FP32
     float wv[E];
     if constexpr (WTAB) {
       const float* __restrict__ w = wlut + (long)r * mlut;

@@ -6,7 +6,7 @@
 //                   packed field z = rec + i*ion (both r2c of :290-291 in one
 //                   complex transform).
 //   k_cols          forward along j (per slice), inverse along j (per radius).
-//   k_filter_i      per radius batch: forward along i, then for each radius
+//   k_filter_tab    per radius batch: forward along i, then for each radius
 //                   the top-hat filter (:305-322) and the inverse along i.
 //   k_inv_rows_crit per radius: inverse along p and the bubble-centre test
 //                   (:327-352, :437-438); centres record the ball bound of
@@ -308,8 +308,9 @@ __global__ __launch_bounds__(256) void k_w_table(int n, const float2* __restrict
 // Sides 256 and 512 hold 16 values per thread: at 512 two blocks of 512
 // threads share a CU (78 KiB of LDS, 128 VGPRs each) and fill each other's
 // exchange barriers.
-// Bound: the stores (512^3: 50.5 GB per slice, with the table's 6.4 GB 5.2
-// TB/s).  512^3, 47 radii, per slice: 14.2 ms with the weights evaluated in
+// Bound: five exchange barriers a radius at 16 waves per CU; neither limit is reached
+// (512^3, 47 radii: 50.5 GB written and 7.5 GB read at 4.7-5.2 TB/s, VALU 51-53%
+// busy).  512^3, 47 radii, per slice: 14.2 ms with the weights evaluated in
 // the loop (a third of its VALU instructions), twiddle loads in it and two
 // lines per 1024-thread block; 17.9 ms with a table in folded order (half
 // cache lines); 14.8 ms with this one; 13.1 ms with the buffer's tiles ordered
@@ -431,8 +432,10 @@ __global__ __launch_bounds__(TILE*(L / Plan<L>::E)) void k_filter_lut(
 // the largest radius -- no atomics and no reads of the map.  A row's threads
 // sit in one wave, so the exchanges need no block barrier; the next radius is
 // loaded during the transform, and the twiddles stay in registers (a load of
-// them would wait for that prefetch).  Bound: HBM reads -- 512^3, 16 radii
-// 4.55 -> 2.62 ms per launch (6.4 TB/s), 256^3 0.42 -> 0.29 ms.  dbg (nullable)
+// them would wait for that prefetch).  Bound: near both limits -- 512^3, 47 radii
+// 8.4-9.0 ms, 5.6-6.0 TB/s of reads (a read-only kernel 6.8) with the VALU 85% busy
+// (93% with 16 values per thread).  16 radii a launch, before and after the
+// prefetch: 4.55 -> 2.62 ms, 256^3 0.42 -> 0.29 ms.  dbg (nullable)
 // receives the unscaled filtered pairs, keep (nullable) the pairs as
 // computed (N^3 rec_R, s N^3 ion_R), for the differentiable mode's backward.
 // ------------------------------------------------------------------------
@@ -510,8 +513,9 @@ __global__ __launch_bounds__(256) void k_inv_rows_crit(const float2* __restrict_
 // phase: TPL threads per row in one wave, as k_inv_rows_crit; rows SR floats
 // apart (SR = 8 mod 32: the four rows of a half wave fall into disjoint banks).
 // Up to 128 a plane fits the 160 KiB of LDS and the registers of one block; at
-// 192 it no longer does.  Bound: LDS exchanges and VALU (one block per CU at
-// 128).  Against separate j and p passes, 16 radii: 128^3 0.124 -> 0.078 ms,
+// 192 it no longer does.  Bound: at 128 the barriers of the exchanges, one block of
+// 16 waves per CU (VALU 53%, LDS 22% busy, 2.8 TB/s); at 64 the launch's own length
+// (VALU 35%, 2.9 TB/s in 18 us).  Against separate j and p passes, 16 radii: 128^3 0.124 -> 0.078 ms,
 // 64^3 (11 radii per launch, 128 blocks walking the radii) 0.049 -> 0.013 ms.
 // ------------------------------------------------------------------------
 template <int L>
@@ -824,11 +828,13 @@ __host__ __device__ constexpr int dt_col_floats(int n) { return n + n / 8 + 1; }
 // QMAX >= a.q: the per-lane result array of the line pass.  The last tile
 // of a row may be partial (n a multiple of 8): its missing columns load as
 // empty (-1) lines and are not stored.
-// Bound by chains of dependent LDS reads: 8 waves a block keep the CU's wave slots
-// full (the LDS of the larger sides leaves room for 4 blocks), 4 left them half
-// empty: 512^3 0.70-0.77 -> 0.57-0.59 ms a pass, 600^3 1.6-1.7 -> 1.2-1.3; 16 were
-// slower from 96 up (512^3 0.66-0.71).  With one block or less per CU (up to 64) a wave per
-// column: 64^3 11-12 -> 8 us (8 waves: 9).
+// Bound by chains of dependent LDS reads until 8 waves a block fill the CU's wave
+// slots (the LDS of the larger sides leaves room for 4 blocks), then by VALU issue;
+// 4 waves left the slots half empty.  The balls' reach sets the work: at a mean x_HII
+// of 0.5 0.85 -> 0.73 ms a pass at 512^3 (47 radii), 2.5 -> 2.0 at 600^3 (48 radii).
+// 16 waves were slower from 96 up (a 512^3 box of smaller balls: 8 waves 0.57-0.59,
+// 16 waves 0.66-0.71).  With one block or less per CU (up to 64) a wave per column:
+// 64^3 11-12 -> 7-8 us (8 waves: 9).
 template <int QMAX>
 __global__ __launch_bounds__(1024) void k_dt_tile(DtArgs a, int axis, const int* in, int* out) {
   extern __shared__ int sm[];

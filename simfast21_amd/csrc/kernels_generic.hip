@@ -570,9 +570,9 @@ __global__ __launch_bounds__(gen_threads(L, gen_row(L)) * gen_row(L)) void k_gen
 // smaller ones take 142-153, and spill at 128: 480^3 11.3 ms against 7.7).
 // dbg (one radius): the unscaled pairs in natural order, the values the test
 // saw.
-// Bound by its VALU and LDS work at 3-4 waves per SIMD: 600^3, 48 radii 23.5 ms
-// for 83 GB (3.5 TB/s; one radius per launch, no prefetch: 28.7), 480^3 7.7 ms
-// (5.3 TB/s).
+// Bound by VALU issue, 81% busy, and the lines it reads: 600^3, 48 radii 23-23.5 ms
+// for 83 GB, 3.5 TB/s (one radius per launch, no prefetch: 28.7), where half lines
+// make it fetch 1.6 times that, 5.1 TB/s; 480^3, whole lines, 7.7 ms (5.3 TB/s).
 template <int L>
 __global__ __launch_bounds__(gen_row_threads(L)* gen_block_rows(L),
                              gen_row_threads(L) * gen_block_rows(L) > 256 ? 4 : 1) void k_gen_crit(
@@ -649,8 +649,8 @@ __global__ __launch_bounds__(gen_row_threads(L)* gen_block_rows(L),
 // plane in one block, 8 threads per line, the plane in LDS between the stages
 // (element (j, p) at j SR + p).  blockIdx.y: groups of rper radii (wmap by
 // atomic maximum when there are several).  Reads the buffer once instead of
-// three accesses: 120^3, 33 radii 0.286 ms, one launch (the LDS exchanges bound
-// it); with the separate passes of one radius each 0.9 ms and 66 launches.
+// three accesses: 120^3, 33 radii 0.28 ms, one launch, bound by the barriers of its
+// exchanges, one block of 15 waves per CU (VALU 34%, LDS 10% busy, 1.8 TB/s); with the separate passes of one radius each 0.9 ms and 66 launches.
 template <int L>
 struct GenPlaneCfg {
   static constexpr int T = 8;

@@ -122,8 +122,9 @@ __global__ void k_fill_value(float* __restrict__ p, float value, long count) {
 // block's LDS the deposits are added there and every touched cell then takes
 // one global atomic, in rows of consecutive addresses -- about 3 per source
 // cell instead of 8.  The LDS sums are FP64: an FP32 LDS atomic takes 193
-// cycles a wave here, an FP64 one 9.  A tile whose cells scatter farther (or
-// hold a NaN) deposits directly.  Blocks stay and take one tile after another,
+// cycles a wave here, an FP64 one 9.  A tile whose cells scatter farther
+// deposits directly (a NaN position truncates to cell 0, with NaN weights, on
+// either way).  Blocks stay and take one tile after another,
 // the next one's velocities loaded while this one is added up.  512^3,
 // displacements of 1.1 cells rms: 24.7 ms direct, 6.1 with FP32 sums in tiles of
 // 16 x 16 x 32, 2.1 this way (2.5 with a block per tile).  Tried and slower: tiles by

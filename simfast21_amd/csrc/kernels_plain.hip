@@ -360,7 +360,9 @@ namespace sf21 {
 // 16 lanes, where the neighbours' values come with the vector operation; over
 // the wave they cost 21 LDS permutes a chunk.  256^3: 0.58 ms (every mode added
 // three LDS atomics to a few addresses, and one block then read 2048 partials
-// in turn) -> 0.057 over the wave -> 0.038 ms.  Bound: the read of the spectrum.
+// in turn) -> 0.057 over the wave -> 0.038 ms with the final sums (0.030 alone).  Bound:
+// the vector work of the segmented sums (256^3: VALU 49% busy, 2.4 TB/s of reads;
+// 512^3 0.42 ms).
 // ------------------------------------------------------------------------
 constexpr int kPkMaxBins = 64;
 
