@@ -296,7 +296,8 @@ int sf21_hii_filtered_dev(sf21_hii_ctx *ctx, const float *a, const float *b, con
  * transforms) have one choice: which column passes (along j, along i) deal
  * runs of consecutive blocks to one XCD (sf21_hii_line_order); the four
  * masks are timed and the winner is cached the same way.  Every choice
- * changes launch shapes or block order only: the results are identical. */
+ * changes launch shapes or block order only: a slice's results are identical
+ * (the differentiable backward's sums are grouped by the radius batch). */
 int sf21_hii_autotune(sf21_hii_ctx *ctx, const float *a, const float *b, const float *c,
                       double z, const char *cache_path, double *best_ms);
 /* Current choices: filter tile, radius batch, top-hat weights (1 FP32, 2

@@ -306,9 +306,9 @@ __global__ __launch_bounds__(256) void k_w_table(int n, const float2* __restrict
 // the second reads them from its L2.  blockIdx.y: groups of rper radii, so
 // that small boxes fill the GPU.
 // Sides 256 and 512 hold 16 values per thread: at 512 two blocks of 512
-// threads share a CU (78 KiB of LDS, 128 VGPRs each) and fill each other's
+// threads share a CU (76 KiB of LDS, 128 VGPRs each) and fill each other's
 // exchange barriers.
-// Bound: five exchange barriers a radius at 16 waves per CU; neither limit is reached
+// Bound: four exchange barriers a radius at 16 waves per CU; neither limit is reached
 // (512^3, 47 radii: 50.5 GB written and 7.5 GB read at 4.7-5.2 TB/s, VALU 51-53%
 // busy).  512^3, 47 radii, per slice: 14.2 ms with the weights evaluated in
 // the loop (a third of its VALU instructions), twiddle loads in it and two
